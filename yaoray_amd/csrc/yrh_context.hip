@@ -35,28 +35,35 @@ int CheckStackOverflow(yrh_context* ctx) {
 
 namespace {
 
-template <typename T>
-int Upload(yrh_context* ctx, DevBuf& buf, const std::vector<T>& host) {
-    buf.reset();
-    const size_t bytes = std::max<size_t>(host.size() * sizeof(T), 16);
-    int rc = CheckHip(ctx, hipMalloc(&buf.ptr, bytes), "hipMalloc");
-    if (rc != YRH_OK) return rc;
-    buf.bytes = bytes;
-    if (!host.empty()) {
-        rc = yrh_copy_to_device(ctx, buf.ptr, host.data(), host.size() * sizeof(T));
-    }
-    return rc;
-}
-
+// A packed tree (or several): interior nodes and primitive slots. Node codes
+// hold an interior node's index, or kLeafBit | a slot's index, until
+// ResolveCode turns the indices into arena units.
 struct PackedBvh {
     std::vector<DevNode> nodes;
-    std::vector<float4> slots;
-    std::vector<int32_t> leaf_count;
+    std::vector<float4> slots;        // three per slot
+    std::vector<int32_t> slot_source;  // per slot: its position in primitive_indices
     int32_t root_code = 0;
     float root_lo[3] = {0, 0, 0};
     float root_hi[3] = {0, 0, 0};
     bool empty = true;
 };
+
+int32_t ResolveCode(int32_t code, int64_t node_base, int64_t leaf_base, int32_t slot_units, int32_t leaf_bits) {
+    if (code >= 0) return static_cast<int32_t>((node_base + code) * kNodeUnits);
+    return leaf_bits | static_cast<int32_t>(leaf_base + static_cast<int64_t>(code & ~kLeafBit) * slot_units);
+}
+
+float IntBits(int32_t v) {
+    float f;
+    std::memcpy(&f, &v, 4);
+    return f;
+}
+
+int32_t FloatBits(float v) {
+    int32_t i;
+    std::memcpy(&i, &v, 4);
+    return i;
+}
 
 // Checks one reference BVH's arrays (child and leaf ranges) and that its
 // declared max_depth covers the tree: the traversal stack is sized from the
@@ -146,63 +153,71 @@ int ValidateGeometry(const yrh_geometry_desc* g, std::string& error) {
     return YRH_OK;
 }
 
-// Validates one reference BVH and appends its repacked form to `out`, rebasing
-// node indices by out.nodes.size() and slots by out.slots.size() / 3.
-// `slot_payload(slot, prim)` writes the three float4 of a slot.
+// Validates one reference BVH and appends its repacked form to `out`: interior
+// nodes in the reference's order, and each leaf's slots one after another
+// (leaves may share primitives). `slot_payload(prim, dst)` writes the three
+// float4 of a slot; the second one's .w is the leaf-end mark, set here.
 template <typename SlotFn>
 bool PackBvh(const yrh_bvh_desc& bvh, PackedBvh& out, std::string& error, SlotFn&& slot_payload) {
-    const int32_t node_base = static_cast<int32_t>(out.nodes.size());
-    const int64_t slot_base = static_cast<int64_t>(out.leaf_count.size());
     if (!ValidateBvh(bvh, error)) return false;
+    const int64_t slot_base = static_cast<int64_t>(out.slot_source.size());
     if (slot_base + bvh.primitive_index_count > kMaxSlot) {
         error = "too many BVH primitive slots for the device layout";
         return false;
     }
-    const auto code_of = [&](int32_t node) -> int32_t {
-        const yrh_bvh_node& n = bvh.nodes[node];
-        if (n.primitive_count > 0) {
-            return PackLeaf(static_cast<int32_t>(slot_base) + n.payload_offset, n.primitive_count);
-        }
-        return node_base + node;
-    };
-    out.nodes.resize(out.nodes.size() + static_cast<size_t>(bvh.node_count));
-    for (int32_t i = 0; i < bvh.node_count; ++i) {
-        const yrh_bvh_node& n = bvh.nodes[i];
-        DevNode& rec = out.nodes[static_cast<size_t>(node_base + i)];
-        if (n.primitive_count > 0) {
-            rec.a = make_float4(0, 0, 0, 0);
-            rec.b = rec.a;
-            rec.c = rec.a;
-            rec.d = make_int4(code_of(i), 0, 0, 0);
-            continue;
-        }
-        const yrh_bvh_node& l = bvh.nodes[i + 1];
-        const yrh_bvh_node& r = bvh.nodes[n.payload_offset];
-        rec.a = make_float4(l.bounds_min[0], l.bounds_min[1], l.bounds_min[2], l.bounds_max[0]);
-        rec.b = make_float4(l.bounds_max[1], l.bounds_max[2], r.bounds_min[0], r.bounds_min[1]);
-        rec.c = make_float4(r.bounds_min[2], r.bounds_max[0], r.bounds_max[1], r.bounds_max[2]);
-        rec.d = make_int4(code_of(i + 1), code_of(n.payload_offset), 0, 0);
-    }
-    out.slots.resize(out.slots.size() + 3 * static_cast<size_t>(bvh.primitive_index_count));
-    out.leaf_count.resize(out.leaf_count.size() + static_cast<size_t>(bvh.primitive_index_count), 0);
+    std::vector<float4> payload(3 * static_cast<size_t>(bvh.primitive_index_count));
     for (int32_t s = 0; s < bvh.primitive_index_count; ++s) {
         const int32_t p = bvh.primitive_indices[s];
         if (p < 0 || p >= bvh.primitive_count) {
             error = "BVH primitive index out of bounds";
             return false;
         }
-        float4* dst = &out.slots[3 * static_cast<size_t>(slot_base + s)];
-        if (!slot_payload(bvh.primitives[p], dst, error)) return false;
+        if (!slot_payload(bvh.primitives[p], &payload[3 * static_cast<size_t>(s)], error)) return false;
     }
+    std::vector<int32_t> code(static_cast<size_t>(bvh.node_count));
+    int64_t interior = static_cast<int64_t>(out.nodes.size());
+    int64_t slots = slot_base;
     for (int32_t i = 0; i < bvh.node_count; ++i) {
         const yrh_bvh_node& n = bvh.nodes[i];
-        if (n.primitive_count > kLeafCountEscape) {
-            out.leaf_count[static_cast<size_t>(slot_base + n.payload_offset)] = n.primitive_count;
+        if (n.primitive_count > 0) {
+            code[static_cast<size_t>(i)] = kLeafBit | static_cast<int32_t>(slots);
+            slots += n.primitive_count;
+        } else {
+            code[static_cast<size_t>(i)] = static_cast<int32_t>(interior++);
         }
+        if (kNodeUnits * interior + kSlotUnits * slots > kMaxUnits) {
+            error = "too many BVH primitive slots for the device layout";
+            return false;
+        }
+    }
+    out.nodes.resize(static_cast<size_t>(interior));
+    out.slots.reserve(3 * static_cast<size_t>(slots));
+    out.slot_source.reserve(static_cast<size_t>(slots));
+    for (int32_t i = 0; i < bvh.node_count; ++i) {
+        const yrh_bvh_node& n = bvh.nodes[i];
+        if (n.primitive_count > 0) {
+            for (int32_t k = 0; k < n.primitive_count; ++k) {
+                const int32_t s = n.payload_offset + k;
+                const float4* src = &payload[3 * static_cast<size_t>(s)];
+                const float last = IntBits(k + 1 == n.primitive_count ? 1 : 0);
+                out.slots.push_back(src[0]);
+                out.slots.push_back(make_float4(src[1].x, src[1].y, src[1].z, last));
+                out.slots.push_back(src[2]);
+                out.slot_source.push_back(s);
+            }
+            continue;
+        }
+        const yrh_bvh_node& l = bvh.nodes[i + 1];
+        const yrh_bvh_node& r = bvh.nodes[n.payload_offset];
+        DevNode& rec = out.nodes[static_cast<size_t>(code[static_cast<size_t>(i)])];
+        rec.a = make_float4(l.bounds_min[0], l.bounds_min[1], l.bounds_min[2], l.bounds_max[0]);
+        rec.b = make_float4(l.bounds_max[1], l.bounds_max[2], r.bounds_min[0], r.bounds_min[1]);
+        rec.c = make_float4(r.bounds_min[2], r.bounds_max[0], r.bounds_max[1], r.bounds_max[2]);
+        rec.d = make_int4(code[static_cast<size_t>(i) + 1], code[static_cast<size_t>(n.payload_offset)], 0, 0);
     }
     if (bvh.node_count > 0) {
         out.empty = false;
-        out.root_code = code_of(0);
+        out.root_code = code[0];
         for (int k = 0; k < 3; ++k) {
             out.root_lo[k] = bvh.nodes[0].bounds_min[k];
             out.root_hi[k] = bvh.nodes[0].bounds_max[k];
@@ -211,7 +226,7 @@ bool PackBvh(const yrh_bvh_desc& bvh, PackedBvh& out, std::string& error, SlotFn
     return true;
 }
 
-// Triangle slot: (p0, flat id bits) (e1, mesh primitive bits) (e2, local triangle bits).
+// Triangle slot: (p0, flat id bits) (e1, 0) (e2, 0).
 // A reference triangle that its traversal would skip (bad handle or index,
 // bvh_traversal.cpp:59-76) becomes a zero-area slot, which the |det| < 1e-8
 // test rejects, so it is counted but never hit, as in the reference.
@@ -219,20 +234,16 @@ struct TriangleSlotWriter {
     const yrh_geometry_desc* g;
     bool operator()(const yrh_bvh_primitive& prim, float4* dst, std::string& error) const {
         if (prim.kind == 1) {
-            // Sphere slot: (centre, -2 - sphere) (radius, 0, 0, -1) (0, 0, 0, -1).
+            // Sphere slot: (centre, -2 - sphere) (radius, 0, 0, 0) (0, 0, 0, 0).
             // A bad handle (skipped by the reference, bvh_traversal.cpp:130-133)
             // gets a NaN centre: counted, never hit.
             const bool ok = prim.sphere >= 0 && prim.sphere < g->sphere_count;
             const float nan = std::numeric_limits<float>::quiet_NaN();
             const yrh_sphere* sp = ok ? &g->spheres[prim.sphere] : nullptr;
-            const int32_t id = -2 - (ok ? prim.sphere : 0);
-            float fid, fneg;
-            const int32_t neg = -1;
-            std::memcpy(&fid, &id, 4);
-            std::memcpy(&fneg, &neg, 4);
+            const float fid = IntBits(-2 - (ok ? prim.sphere : 0));
             dst[0] = ok ? make_float4(sp->center[0], sp->center[1], sp->center[2], fid) : make_float4(nan, nan, nan, fid);
-            dst[1] = make_float4(ok ? sp->radius : nan, 0.0f, 0.0f, fneg);
-            dst[2] = make_float4(0.0f, 0.0f, 0.0f, fneg);
+            dst[1] = make_float4(ok ? sp->radius : nan, 0.0f, 0.0f, 0.0f);
+            dst[2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             return true;
         }
         if (prim.kind != 0) {
@@ -266,16 +277,9 @@ struct TriangleSlotWriter {
                 e2[c] = p[2][c] - p[0][c];
             }
         }
-        int32_t id = prim.flat_triangle_index;
-        int32_t mesh = prim.mesh_primitive;
-        int32_t local = prim.local_triangle;
-        float fid, fmesh, flocal;
-        std::memcpy(&fid, &id, 4);
-        std::memcpy(&fmesh, &mesh, 4);
-        std::memcpy(&flocal, &local, 4);
-        dst[0] = make_float4(p[0][0], p[0][1], p[0][2], fid);
-        dst[1] = make_float4(e1[0], e1[1], e1[2], fmesh);
-        dst[2] = make_float4(e2[0], e2[1], e2[2], flocal);
+        dst[0] = make_float4(p[0][0], p[0][1], p[0][2], IntBits(prim.flat_triangle_index));
+        dst[1] = make_float4(e1[0], e1[1], e1[2], 0.0f);
+        dst[2] = make_float4(e2[0], e2[1], e2[2], 0.0f);
         return true;
     }
 };
@@ -496,7 +500,9 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
     DevGeometry& geo = ctx->geo;
     std::string error;
     TriangleSlotWriter writer{g};
-    PackedBvh packed;
+    PackedBvh packed;  // the flat BVH, or every BLAS
+    PackedBvh tl;      // two-level: the TLAS
+    std::vector<DevInstanceSlot> instances;
 
     if (g->accel_kind == YRH_ACCEL_FLAT) {
         if (!PackBvh(g->flat, packed, error, writer)) return Fail(ctx, YRH_E_INVALID_ARGUMENT, error);
@@ -509,26 +515,12 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
         std::vector<DevBlasRoot> roots(static_cast<size_t>(g->blas_count));
         int32_t blas_depth = 1;
         for (int32_t b = 0; b < g->blas_count; ++b) {
-            PackedBvh one;
-            const size_t node_base = packed.nodes.size();
-            const size_t slot_base = packed.leaf_count.size();
-            // Pack into the shared arrays by pre-seeding sizes.
-            one.nodes.swap(packed.nodes);
-            one.slots.swap(packed.slots);
-            one.leaf_count.swap(packed.leaf_count);
-            const bool ok = PackBvh(g->blases[b], one, error, writer);
-            packed.nodes.swap(one.nodes);
-            packed.slots.swap(one.slots);
-            packed.leaf_count.swap(one.leaf_count);
-            if (!ok) return Fail(ctx, YRH_E_INVALID_ARGUMENT, error);
-            if (one.empty) return Fail(ctx, YRH_E_INVALID_ARGUMENT, "empty BLAS");
-            (void)node_base;
-            (void)slot_base;
-            int32_t code = one.root_code;
-            float fcode;
-            std::memcpy(&fcode, &code, 4);
-            roots[static_cast<size_t>(b)].lo = make_float4(one.root_lo[0], one.root_lo[1], one.root_lo[2], fcode);
-            roots[static_cast<size_t>(b)].hi = make_float4(one.root_hi[0], one.root_hi[1], one.root_hi[2], 0.0f);
+            packed.empty = true;
+            if (!PackBvh(g->blases[b], packed, error, writer)) return Fail(ctx, YRH_E_INVALID_ARGUMENT, error);
+            if (packed.empty) return Fail(ctx, YRH_E_INVALID_ARGUMENT, "empty BLAS");
+            DevBlasRoot& root = roots[static_cast<size_t>(b)];
+            root.lo = make_float4(packed.root_lo[0], packed.root_lo[1], packed.root_lo[2], IntBits(packed.root_code));
+            root.hi = make_float4(packed.root_hi[0], packed.root_hi[1], packed.root_hi[2], 0.0f);
             blas_depth = std::max(blas_depth, g->blases[b].max_depth);
         }
         // TLAS: slots resolve primitive_indices -> tlas primitive -> instance.
@@ -536,13 +528,7 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
         if (t.primitive_index_count > 0 && (t.primitive_indices == nullptr || g->tlas_primitives == nullptr)) {
             return Fail(ctx, YRH_E_INVALID_ARGUMENT, "TLAS arrays missing");
         }
-        PackedBvh tl;
-        std::vector<int32_t> slot_instance;
-        yrh_bvh_desc tdesc = t;
-        tdesc.primitives = nullptr;
-        tdesc.primitive_count = g->tlas_primitive_count;
-        // Reuse PackBvh for nodes/codes with a slot writer that records instances.
-        // Per TLAS slot: an instance index (>= 0) or -2 - sphere index.
+        // Per primitive_indices position: an instance index (>= 0) or -2 - sphere index.
         std::vector<int32_t> resolved(static_cast<size_t>(std::max(0, t.primitive_index_count)), -1);
         for (int32_t s = 0; s < t.primitive_index_count; ++s) {
             const int32_t p = t.primitive_indices[s];
@@ -561,7 +547,10 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
             if (bi < 0 || bi >= g->blas_count) return Fail(ctx, YRH_E_INVALID_ARGUMENT, "instance BLAS out of bounds");
             resolved[static_cast<size_t>(s)] = tp.instance;
         }
+        // PackBvh gives the nodes and, per slot, its position; the instance
+        // slots are filled from those.
         std::vector<yrh_bvh_primitive> dummy(static_cast<size_t>(std::max(1, g->tlas_primitive_count)));
+        yrh_bvh_desc tdesc = t;
         tdesc.primitives = dummy.data();
         tdesc.primitive_count = static_cast<int32_t>(dummy.size());
         const auto no_slot = [](const yrh_bvh_primitive&, float4* dst, std::string&) {
@@ -569,50 +558,73 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
             return true;
         };
         if (!PackBvh(tdesc, tl, error, no_slot)) return Fail(ctx, YRH_E_INVALID_ARGUMENT, error);
-        std::vector<DevInstanceSlot> slots(resolved.size());
-        for (size_t s = 0; s < resolved.size(); ++s) {
-            const int32_t i = resolved[s];
+        const int64_t slot_base = static_cast<int64_t>(packed.nodes.size() + tl.nodes.size()) * kNodeUnits;
+        instances.resize(tl.slot_source.size());
+        for (size_t s = 0; s < instances.size(); ++s) {
+            const int32_t i = resolved[static_cast<size_t>(tl.slot_source[s])];
+            const int32_t last = FloatBits(tl.slots[3 * s + 1].w) != 0 ? kInstanceBit : 0;
+            DevInstanceSlot& d = instances[s];
             if (i <= -2) {
                 // TLAS sphere slot: r0 = (centre, radius), hi.w = -2 - sphere.
                 const yrh_sphere& sp = g->spheres[-2 - i];
-                float fi;
-                std::memcpy(&fi, &i, 4);
-                DevInstanceSlot& d = slots[s];
                 d.r0 = make_float4(sp.center[0], sp.center[1], sp.center[2], sp.radius);
-                d.r1 = d.r2 = d.lo = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                d.hi = make_float4(0.0f, 0.0f, 0.0f, fi);
+                d.r1 = d.r2 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                d.lo = make_float4(0.0f, 0.0f, 0.0f, IntBits(last));
+                d.hi = make_float4(0.0f, 0.0f, 0.0f, IntBits(i));
                 continue;
             }
             const float* m = g->instances[i].world_to_object;
             const DevBlasRoot& root = roots[static_cast<size_t>(g->instances[i].blas_index)];
-            DevInstanceSlot& d = slots[s];
             d.r0 = make_float4(m[0], m[4], m[8], m[12]);
             d.r1 = make_float4(m[1], m[5], m[9], m[13]);
             d.r2 = make_float4(m[2], m[6], m[10], m[14]);
-            float fi;
-            std::memcpy(&fi, &i, 4);
             d.lo = root.lo;
-            d.hi = make_float4(root.hi.x, root.hi.y, root.hi.z, fi);
+            d.lo.w = IntBits(ResolveCode(FloatBits(root.lo.w), 0, slot_base, kSlotUnits, kLeafBit) | last);
+            d.hi = make_float4(root.hi.x, root.hi.y, root.hi.z, IntBits(i));
         }
-        geo.instance_count = g->instance_count;
-        geo.blas_count = g->blas_count;
-        geo.root_code = tl.root_code;
-        std::memcpy(geo.root_lo, tl.root_lo, sizeof(geo.root_lo));
-        std::memcpy(geo.root_hi, tl.root_hi, sizeof(geo.root_hi));
-        geo.empty = tl.empty;
         geo.stack_capacity = std::max(1, t.max_depth) + blas_depth + 3;
-        if ((rc = Upload(ctx, geo.tlas_nodes, tl.nodes)) != YRH_OK) return rc;
-        if ((rc = Upload(ctx, geo.tlas_leaf_count, tl.leaf_count)) != YRH_OK) return rc;
-        if ((rc = Upload(ctx, geo.instance_slots, slots)) != YRH_OK) return rc;
     } else {
         return Fail(ctx, YRH_E_INVALID_ARGUMENT, "unknown acceleration kind");
     }
 
-    if (g->accel_kind == YRH_ACCEL_FLAT) {
-        geo.root_code = packed.root_code;
-        std::memcpy(geo.root_lo, packed.root_lo, sizeof(geo.root_lo));
-        std::memcpy(geo.root_hi, packed.root_hi, sizeof(geo.root_hi));
-        geo.empty = packed.empty;
+    // The arena: nodes (BLASes or the flat tree, then the TLAS), primitive
+    // slots, instance slots; indices become units.
+    {
+        const int64_t tlas_base = static_cast<int64_t>(packed.nodes.size());
+        const int64_t nodes = tlas_base + static_cast<int64_t>(tl.nodes.size());
+        const int64_t slot_base = nodes * kNodeUnits;
+        const int64_t inst_base = slot_base + static_cast<int64_t>(packed.slots.size());
+        const int64_t units = inst_base + static_cast<int64_t>(instances.size()) * kInstanceUnits;
+        if (units > kMaxUnits) return Fail(ctx, YRH_E_INVALID_ARGUMENT, "too many BVH primitive slots for the device layout");
+        const int32_t tlas_leaf = kLeafBit | kInstanceBit;
+        for (DevNode& n : packed.nodes) {
+            n.d.x = ResolveCode(n.d.x, 0, slot_base, kSlotUnits, kLeafBit);
+            n.d.y = ResolveCode(n.d.y, 0, slot_base, kSlotUnits, kLeafBit);
+        }
+        for (DevNode& n : tl.nodes) {
+            n.d.x = ResolveCode(n.d.x, tlas_base, inst_base, kInstanceUnits, tlas_leaf);
+            n.d.y = ResolveCode(n.d.y, tlas_base, inst_base, kInstanceUnits, tlas_leaf);
+        }
+        const bool two = g->accel_kind == YRH_ACCEL_TWO_LEVEL;
+        const PackedBvh& top = two ? tl : packed;
+        geo.empty = top.empty;
+        geo.root_code = two ? ResolveCode(tl.root_code, tlas_base, inst_base, kInstanceUnits, tlas_leaf)
+                            : ResolveCode(packed.root_code, 0, slot_base, kSlotUnits, kLeafBit);
+        std::memcpy(geo.root_lo, top.root_lo, sizeof(geo.root_lo));
+        std::memcpy(geo.root_hi, top.root_hi, sizeof(geo.root_hi));
+        const size_t bytes = static_cast<size_t>(std::max<int64_t>(units, 1)) * sizeof(float4);
+        if ((rc = CheckHip(ctx, hipMalloc(&geo.arena.ptr, bytes), "hipMalloc")) != YRH_OK) return rc;
+        geo.arena.bytes = bytes;
+        float4* base = geo.arena.as<float4>();
+        if ((rc = yrh_copy_to_device(ctx, base, packed.nodes.data(), packed.nodes.size() * sizeof(DevNode))) != YRH_OK ||
+            (rc = yrh_copy_to_device(ctx, base + tlas_base * kNodeUnits, tl.nodes.data(),
+                                     tl.nodes.size() * sizeof(DevNode))) != YRH_OK ||
+            (rc = yrh_copy_to_device(ctx, base + slot_base, packed.slots.data(),
+                                     packed.slots.size() * sizeof(float4))) != YRH_OK ||
+            (rc = yrh_copy_to_device(ctx, base + inst_base, instances.data(),
+                                     instances.size() * sizeof(DevInstanceSlot))) != YRH_OK) {
+            return rc;
+        }
     }
     geo.accel_kind = g->accel_kind;
     // Sphere slots exist if any flat-BVH or TLAS primitive is a sphere (an
@@ -627,10 +639,6 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
             geo.has_spheres = g->tlas_primitives[k].kind != 0;
         }
     }
-    geo.slot_count = static_cast<int64_t>(packed.leaf_count.size());
-    if ((rc = Upload(ctx, geo.nodes, packed.nodes)) != YRH_OK) return rc;
-    if ((rc = Upload(ctx, geo.slots, packed.slots)) != YRH_OK) return rc;
-    if ((rc = Upload(ctx, geo.leaf_count, packed.leaf_count)) != YRH_OK) return rc;
     if ((rc = UploadSurfaceGeometry(ctx, g)) != YRH_OK) return rc;
     geo.loaded = true;
     return YRH_OK;

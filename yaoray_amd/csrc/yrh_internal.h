@@ -1,20 +1,24 @@
 // Internal declarations shared by the libyrh translation units.
 //
-// Device layout of the acceleration structure (MI355X / gfx950):
+// Device layout of the acceleration structure (MI355X / gfx950): one arena of
+// 16-byte units per scene, so every record is named by its unit.
 //   * A binary BVH is the reference's own tree (include/yaoray/accel/bvh.hpp:34-47),
 //     repacked so that an interior node carries both child boxes: one 64-byte
 //     record (four 16-byte loads issued together) instead of two dependent
 //     32-byte node reads per interior step. Visit order, box arithmetic and the
-//     node_tests counter are unchanged.
-//   * A child is named by a 32-bit "code": >= 0 is an interior node index,
-//     < 0 a leaf: bit 31 set, bits 27..30 = count-1 (15 = escape, count read from
-//     leaf_count[first]), bits 0..26 = first primitive slot.
-//   * Primitive slots follow the leaf order of primitive_indices; each slot
-//     holds the triangle as (p0, e1 = p1 - p0, e2 = p2 - p0) plus its flat
-//     triangle index: 3 x float4 = 48 bytes, one coalesced fetch per test in
-//     place of the reference's 5-level index chase (bvh_traversal.cpp:59-79).
-//     e1/e2 are the same IEEE subtractions the reference performs per test,
-//     so every intersection is bit-identical.
+//     node_tests counter are unchanged. Only interior nodes have a record
+//     (half of a binary tree's nodes are leaves), in the reference's order.
+//   * A child is named by a 32-bit code: >= 0 is an interior node's unit;
+//     < 0 a leaf: bit 31 set, bits 0..29 the unit of its first slot, bit 30
+//     set for a TLAS leaf (instance slots). kNoRecord names nothing.
+//   * Primitive slots follow the nodes, each leaf's in leaf order; a slot
+//     holds the triangle as (p0, flat triangle index) (e1 = p1 - p0, last)
+//     (e2 = p2 - p0, 0): 48 bytes, one coalesced fetch per test in place of
+//     the reference's 5-level index chase (bvh_traversal.cpp:59-79). `last` is
+//     1 in the leaf's last slot, so a leaf needs no count. e1/e2 are the same
+//     IEEE subtractions the reference performs per test, so every
+//     intersection is bit-identical.
+//   * Instance slots (two-level scenes) come last, 80 bytes each.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -38,13 +42,21 @@ struct StageRange {
     StageRange& operator=(const StageRange&) = delete;
 };
 
-constexpr int kLeafCountEscape = 15;
 // Context work-counter words (yrh_context::work_counter).
 constexpr int kOverflowWord = 2;  // traversal stack overflow flag
 constexpr int kCounterSetBase = 256;
 constexpr int kCounterSetWords = 256;  // 8 ranges x 32 words
 constexpr size_t kWorkCounterBytes = (kCounterSetBase + 2 * kCounterSetWords) * sizeof(uint32_t);
 constexpr int32_t kMaxSlot = (1 << 27) - 1;
+// Arena units (16 bytes): record sizes and the code words that name them.
+constexpr int32_t kNodeUnits = 4;
+constexpr int32_t kSlotUnits = 3;
+constexpr int32_t kInstanceUnits = 5;
+constexpr int32_t kLeafBit = static_cast<int32_t>(0x80000000u);
+constexpr int32_t kInstanceBit = 0x40000000;
+constexpr int32_t kUnitMask = 0x3fffffff;
+constexpr int32_t kNoRecord = 0x7fffffff;
+constexpr int64_t kMaxUnits = int64_t{1} << 30;
 
 struct alignas(16) DevNode {
     float4 a;  // L.min.x L.min.y L.min.z L.max.x
@@ -61,21 +73,16 @@ struct alignas(16) DevBlasRoot {
 };
 
 // One TLAS leaf slot: the instance's world-to-object rows and its BLAS root,
-// so a traversal step into an instance is one 80-byte fetch.
+// so a traversal step into an instance is one 80-byte fetch. The root code's
+// bit 30 is set in the last slot of a leaf.
 struct alignas(16) DevInstanceSlot {
     float4 r0;  // world_to_object m[0], m[4], m[8],  m[12]
     float4 r1;  //                 m[1], m[5], m[9],  m[13]
     float4 r2;  //                 m[2], m[6], m[10], m[14]
-    float4 lo;  // BLAS root box min, w = root code bits
+    float4 lo;  // BLAS root box min, w = root code bits (bit 30: last slot of the leaf)
     float4 hi;  // BLAS root box max, w = instance index bits
 };
 static_assert(sizeof(DevInstanceSlot) == 80, "instance slot record is 80 bytes");
-
-inline int32_t PackLeaf(int32_t first, int32_t count) {
-    const int32_t nib = count <= kLeafCountEscape ? count - 1 : kLeafCountEscape;
-    return static_cast<int32_t>(0x80000000u | (static_cast<uint32_t>(nib) << 27) |
-                                static_cast<uint32_t>(first));
-}
 
 // Device buffer owned by a context.
 struct DevBuf {
@@ -111,22 +118,14 @@ struct DevBuf {
 struct DevGeometry {
     bool loaded = false;
     int accel_kind = YRH_ACCEL_FLAT;
-    // flat BVH, or every BLAS concatenated (node and slot indices rebased)
-    DevBuf nodes;
-    DevBuf slots;       // float4[3 * slot_count]
-    DevBuf leaf_count;  // int32[slot_count], read only for escaped leaves
-    int64_t slot_count = 0;
+    // Interior nodes (flat BVH, or every BLAS and then the TLAS), primitive
+    // slots, instance slots: float4 units.
+    DevBuf arena;
     int32_t root_code = 0;
     float root_lo[3] = {0, 0, 0};
     float root_hi[3] = {0, 0, 0};
     bool empty = true;
     bool has_spheres = false;  // sphere slots exist: launch the traversal variant that tests them
-    // two-level
-    DevBuf tlas_nodes;
-    DevBuf tlas_leaf_count;
-    DevBuf instance_slots;      // DevInstanceSlot per TLAS slot
-    int32_t instance_count = 0;
-    int32_t blas_count = 0;
     int32_t stack_capacity = 0;  // entries needed by the deepest traversal
 };
 

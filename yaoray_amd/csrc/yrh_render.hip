@@ -1643,7 +1643,7 @@ struct ShadowWalk {
         const bool finite = st.z != 0;
         uint32_t occ = 1u;
         bool again = false;
-        bool hit = best.hit;
+        bool hit = best.Hit();
         if (kAlpha && hit && !trav::IsSphereId(best.id) &&
             !(HitAlpha(*S, *L, best.id, inst, best.u, best.v, XYZ(lo), XYZ(ld), best.t, nullptr) >= 0.5f)) {
             // TraceVisibleSurface's alpha skip within this segment
@@ -1804,7 +1804,7 @@ struct AlphaPath {
     __device__ __forceinline__ bool Finish(int32_t ray, const trav::Best& best, int32_t inst, uint32_t, uint32_t,
                                            uint32_t, const float4& lo, const float4& ld, float4& next_org,
                                            float4& next_dir) const {
-        bool hit = best.hit;
+        bool hit = best.Hit();
         if (hit && !trav::IsSphereId(best.id)) {
             const float4* df = diff != nullptr ? diff + 2 * q_path[ray] : nullptr;
             if (!(HitAlpha(*S, *L, best.id, inst, best.u, best.v, XYZ(lo), XYZ(ld), best.t, df) >= 0.5f)) {

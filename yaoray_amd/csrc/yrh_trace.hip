@@ -108,9 +108,7 @@ int PrepareTraceArgs(yrh_context* ctx, const TraceRequest& r, trav::TraceArgs& a
     a.triangle_tests = r.triangle_tests;
     a.sphere_tests = r.sphere_tests;
     a.occluded = r.occluded;
-    a.nodes = g.nodes.as<DevNode>();
-    a.slots = g.slots.as<float4>();
-    a.leaf_count = g.leaf_count.as<int32_t>();
+    a.arena = g.arena.as<float4>();
     a.root_code = g.root_code;
     a.root_lo_x = g.root_lo[0];
     a.root_lo_y = g.root_lo[1];
@@ -119,9 +117,6 @@ int PrepareTraceArgs(yrh_context* ctx, const TraceRequest& r, trav::TraceArgs& a
     a.root_hi_y = g.root_hi[1];
     a.root_hi_z = g.root_hi[2];
     a.empty = g.empty ? 1 : 0;
-    a.tnodes = g.tlas_nodes.as<DevNode>();
-    a.tleaf_count = g.tlas_leaf_count.as<int32_t>();
-    a.instance_slots = g.instance_slots.as<DevInstanceSlot>();
     uint32_t* words = ctx->work_counter.as<uint32_t>();
     if (r.work_counter != nullptr) {
         a.counter = r.work_counter;
