@@ -200,6 +200,26 @@ def two_level_scene():
     return s
 
 
+@pytest.mark.parametrize("shape", [(4, 256), (1, 64), (3, 128)])
+@pytest.mark.parametrize("n", [1, 5, 63, 2047, 2049, 16385, 131072, 131073, 150001])
+def test_every_ray_is_claimed_once(device, n, shape):
+    """Queue lengths around the sizes where rays are dealt by position, spread
+    over more waves than they fill, or claimed from the range counters."""
+    s = Scene.triangles(300, seed=3)
+    s.build_accel()
+    org, d = random_rays(n, seed=21)
+    v, i, p = s.geometry()
+    o = O.trace_flat(v, i, p, s.flat_bvh(), org, d)
+    device.upload_scene(s)
+    device.set_trace_config(*shape)
+    try:
+        assert_same(device.trace_closest(org, d, counters=True), o)
+        g = device.trace_any(org, d)
+    finally:
+        device.set_trace_config(4, 256)
+    assert np.array_equal(g["occluded"].astype(bool), o["triangle"] >= 0)
+
+
 def test_two_level_closest_and_any_match_oracle(device):
     s = two_level_scene()
     v, i, p = s.geometry()

@@ -200,15 +200,15 @@ struct TraceRequest {
     const uint32_t* n_device = nullptr;  // device-resident ray count (read by the kernel)
     int64_t capacity = 0;                // upper bound of *n_device
     int64_t expected = 0;                // typical live count (sizes the grid; 0 = capacity)
-    uint32_t* work_counter = nullptr;    // zeroed ray counter(s) owned by the caller; null = context's
-    int parts = 1;                       // caller's counters: 1, or trav::kParts ranges kPartStride words apart
+    // Zeroed ray counters owned by the caller (trav::kParts, kPartStride words apart); null = context's.
+    uint32_t* work_counter = nullptr;
     float4* hit = nullptr;
     int32_t* instance = nullptr;
     uint32_t* node_tests = nullptr;
     uint32_t* triangle_tests = nullptr;
     uint32_t* sphere_tests = nullptr;
     uint32_t* occluded = nullptr;
-    unsigned long long* totals = nullptr;  // [0] node tests, [1] triangle tests, [2] sphere tests
+    unsigned long long* totals = nullptr;  // test sums (trav::TraceArgs::totals)
     const int32_t* order = nullptr;        // claim position -> ray index (null = identity)
     bool aux = false;                      // on the context's second stream, with its spill region
     // Caller-provided stack spill region (never reallocated): the grid is

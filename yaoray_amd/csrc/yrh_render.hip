@@ -58,15 +58,12 @@ enum Stat : int {
     kStatRays = 0,
     kStatShadow,
     kStatOccluded,
+    kStatNodeTests,  // the trace kernels' sums: [node, triangle, sphere]
     kStatTriTests,
     kStatSphereTests,
-    kStatNodeTests,
     kStatHits,
     kStatMisses,
     kStatBad,
-    kStatTraceNodes,  // scratch totals written by the trace kernels: [node, tri, sphere]
-    kStatTraceTris,
-    kStatTraceSpheres,
     kStatWords,
 };
 // The statistics live in kStatSlots copies kStatStride words (128 B) apart;
@@ -76,6 +73,7 @@ enum Stat : int {
 constexpr int kStatSlots = 64;
 constexpr int kStatStride = 16;
 static_assert(kStatWords <= kStatStride, "statistics words fit a slot");
+static_assert(kStatSlots == trav::kTotalsSlots && kStatStride == trav::kTotalsStride, "the trace kernels add to the slots");
 constexpr size_t kStatBytes = sizeof(unsigned long long) * kStatStride * kStatSlots;
 
 }  // namespace
@@ -853,17 +851,6 @@ __global__ void BeginBounceKernel(uint32_t* counters, int next_queue, int what) 
         if (i >= 2 && i < 2 + trav::kParts) counters[kWorkShadow + (i - 2) * trav::kPartStride] = 0u;
     }
     if ((what & kBeginTrace) && i < trav::kParts) counters[kWorkExtend + i * trav::kPartStride] = 0u;
-}
-
-__global__ void CopyTraceTotalsKernel(unsigned long long* stats) {
-    if (threadIdx.x == 0) {
-        stats[kStatNodeTests] += stats[kStatTraceNodes];
-        stats[kStatTriTests] += stats[kStatTraceTris];
-        stats[kStatSphereTests] += stats[kStatTraceSpheres];
-        stats[kStatTraceNodes] = 0;
-        stats[kStatTraceTris] = 0;
-        stats[kStatTraceSpheres] = 0;
-    }
 }
 
 struct SurfacePoint {
@@ -2292,10 +2279,9 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
         tr.capacity = paths;
         tr.expected = paths;
         tr.work_counter = P.counters + kWorkExtend;
-        tr.parts = trav::kParts;
         tr.hit = P.hits;
         tr.instance = ctx->geo.accel_kind == YRH_ACCEL_TWO_LEVEL ? P.hit_inst : nullptr;
-        tr.totals = P.stats + kStatTraceNodes;
+        tr.totals = P.stats + kStatNodeTests;
         PassView Pk = P;
         if (ctx->geo.accel_kind != YRH_ACCEL_TWO_LEVEL) Pk.hit_inst = nullptr;
         if (depth > 0) Pk.p_diff = nullptr;  // only camera rays carry differentials
@@ -2355,9 +2341,8 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
             sr.capacity = R.shadow_slots * paths;
             sr.expected = paths;  // about one shadow ray per path in flight
             sr.work_counter = P.counters + kWorkShadow;
-            sr.parts = trav::kParts;
-            sr.occluded = P.s_occ;
-            sr.totals = P.stats + kStatTraceNodes;
+                sr.occluded = P.s_occ;
+            sr.totals = P.stats + kStatNodeTests;
             sr.aux = overlap;
             if ((rc = LaunchTrace(ctx, sr)) != YRH_OK) return rc;
         } else {
@@ -2369,9 +2354,8 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
             wr.capacity = R.shadow_slots * paths;
             wr.expected = paths;
             wr.work_counter = P.counters + kWorkShadow;
-            wr.parts = trav::kParts;
-            wr.hit = P.s_trans;  // not written by the walk; LaunchTrace's checks want an output
-            wr.totals = P.stats + kStatTraceNodes;
+                wr.hit = P.s_trans;  // not written by the walk; LaunchTrace's checks want an output
+            wr.totals = P.stats + kStatNodeTests;
             wr.aux = overlap;
             trav::TraceArgs wa;
             int wgrid = 0, wblock = 0;
@@ -2948,9 +2932,9 @@ int yrh_render_stats_read(yrh_context* ctx, yrh_render_stats* stats) {
     stats->rays_traced = w[kStatRays];
     stats->shadow_rays = w[kStatShadow];
     stats->occluded_shadow_rays = w[kStatOccluded];
-    stats->triangle_tests = w[kStatTriTests] + w[kStatTraceTris];
-    stats->sphere_tests = w[kStatSphereTests] + w[kStatTraceSpheres];
-    stats->bvh_node_tests = w[kStatNodeTests] + w[kStatTraceNodes];
+    stats->triangle_tests = w[kStatTriTests];
+    stats->sphere_tests = w[kStatSphereTests];
+    stats->bvh_node_tests = w[kStatNodeTests];
     stats->hits = w[kStatHits];
     stats->misses = w[kStatMisses];
     stats->bad_samples = w[kStatBad];
@@ -3004,7 +2988,6 @@ int yrh_render_pass(yrh_context* ctx, const yrh_render_desc* d) {
     if ((rc = GuidePrepareView(ctx, paths, max_depth, &GV)) != YRH_OK) return rc;
     if ((rc = LaunchPassSequence(ctx, R, P, S, L, GV, paths, max_depth, ctx->render_overlap)) != YRH_OK) return rc;
     hipLaunchKernelGGL(AccumulateKernel, dim3(Grid(npix)), dim3(kBlock), 0, st, P);
-    hipLaunchKernelGGL(CopyTraceTotalsKernel, dim3(1), dim3(64), 0, st, P.stats);
     return CheckHip(ctx, hipGetLastError(), "render pass launch");
 }
 
@@ -3142,7 +3125,6 @@ int yrh_batch_render(yrh_context* ctx, const yrh_batch_desc* d, float* job_ms, i
         for (int32_t occ = 0; occ <= max_occurrence; ++occ) {
             hipLaunchKernelGGL(AccumulateBatchKernel, dim3(Grid(capacity)), dim3(kBlock), 0, st, P, occ);
         }
-        hipLaunchKernelGGL(CopyTraceTotalsKernel, dim3(1), dim3(64), 0, st, P.stats);
         hipLaunchKernelGGL(EndPassKernel, dim3(1), dim3(64), 0, st, P.counters);
         return CheckHip(ctx, hipGetLastError(), "batch pass launch");
     };

@@ -53,15 +53,13 @@ int PrepareTraceArgs(yrh_context* ctx, const TraceRequest& r, trav::TraceArgs& a
                            ? ctx->blocks_per_cu
                            : std::max(1, std::min(8, (160 * 1024) / (lds_levels * block * static_cast<int>(sizeof(int2)))));
     grid = ctx->compute_units * per_cu;
-    const int64_t lanes = static_cast<int64_t>(grid) * block;
-    // Small queues: keep at least 4 rays per lane (the persistent lanes refill
-    // from the counter, so fewer, fuller workgroups drain faster), and never
-    // more lanes than rays.
+    // Never more workgroups than the waves that the queue's rays keep busy.
     const int64_t bound = r.n_device != nullptr ? (r.expected > 0 ? std::min(r.expected, r.capacity) : r.capacity)
                                                 : r.n_host;
-    const int64_t want = std::max<int64_t>(std::min<int64_t>(bound, static_cast<int64_t>(ctx->compute_units) * block),
-                                           (bound + 3) / 4);
-    if (lanes > want) grid = static_cast<int>(std::max<int64_t>(1, (want + block - 1) / block));
+    const int spread_waves = 8 * ctx->compute_units;
+    const int waves_per_group = std::max(1, block / 64);
+    const int64_t waves = trav::RaySource::Waves(bound, spread_waves);
+    grid = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(grid, (waves + waves_per_group - 1) / waves_per_group)));
     const int32_t capacity = g.stack_capacity;
     const int64_t spill_levels = std::max<int64_t>(0, capacity - lds_levels);
     int2* spill_ptr = nullptr;
@@ -121,14 +119,13 @@ int PrepareTraceArgs(yrh_context* ctx, const TraceRequest& r, trav::TraceArgs& a
     if (r.work_counter != nullptr) {
         a.counter = r.work_counter;
         a.next_counter = nullptr;
-        a.parts = r.parts;
     } else {
         // Two sets of per-range counters; each launch zeroes the other set.
         uint32_t* sets = words + kCounterSetBase;
         a.counter = sets + ctx->launch_parity * kCounterSetWords;
         a.next_counter = sets + (1 - ctx->launch_parity) * kCounterSetWords;
-        a.parts = trav::kParts;
     }
+    a.spread_waves = spread_waves;
     a.order = r.order;
     a.overflow = words + kOverflowWord;
     a.spill = spill_ptr != nullptr ? spill_ptr : spill.as<int2>();

@@ -52,13 +52,22 @@ namespace trav {
 constexpr int kMaxLdsStack = 16;  // LDS stack levels per lane, at most (launch option)
 constexpr int kMaxBlock = 256;
 constexpr int kRefillIdleLanes = 32;  // refill once half the wave is idle (swept: 8..56)
+constexpr int kParts = 8;             // claim ranges, one per XCD
+constexpr int kPartStride = 32;       // words between their counters: one cache line each
+// Test sums are kept in copies on cache lines of their own; workgroup b adds
+// to copy b % kTotalsSlots. On one line the 4096 waves of a bounce took 228 us
+// to add theirs, however few rays they had traced.
+constexpr int kTotalsSlots = 64;
+constexpr int kTotalsStride = 16;
 
 struct TraceArgs {
     const float4* org;
     const float4* dir;
     int32_t n;
     const uint32_t* n_device;    // when set, the ray count is read from device memory
-    unsigned long long* totals;  // optional [0] node, [1] triangle, [2] sphere tests of the launch
+    // optional test sums: kTotalsSlots copies kTotalsStride words apart, each
+    // [0] node, [1] triangle, [2] sphere tests
+    unsigned long long* totals;
     // outputs
     float4* hit;
     int32_t* inst_out;
@@ -72,9 +81,9 @@ struct TraceArgs {
     float root_lo_x, root_lo_y, root_lo_z, root_hi_x, root_hi_y, root_hi_z;
     int32_t empty;
     // scheduling
-    uint32_t* counter;       // this launch's ray counter (zero at launch)
-    uint32_t* next_counter;  // the next launch's counter(s), zeroed here (may be null)
-    int32_t parts;           // 1: one counter; kParts: per-range counters kPartStride words apart
+    uint32_t* counter;       // this launch's kParts ray counters, kPartStride words apart (zero at launch)
+    uint32_t* next_counter;  // the next launch's counters, zeroed here (may be null)
+    int32_t spread_waves;    // waves that a short queue is spread over
     const int32_t* order;    // claim position -> ray index (null = identity)
     uint32_t* overflow;      // stack overflow flag
     int2* spill;
@@ -362,6 +371,11 @@ __device__ __forceinline__ int32_t NextSlot(int32_t code, int32_t units, bool la
 
 __device__ __forceinline__ uint64_t LanesBelow(int lane) { return (1ull << lane) - 1ull; }
 
+// Where this workgroup's test sums go.
+__device__ __forceinline__ unsigned long long* TotalsSlot(unsigned long long* totals) {
+    return totals + static_cast<int64_t>(blockIdx.x % kTotalsSlots) * kTotalsStride;
+}
+
 // Wave-level sum of the per-lane test counts (node, triangle, sphere), one
 // atomic per wave and count.
 __device__ __forceinline__ void AddTotals(unsigned long long* totals, uint64_t nt, uint64_t tt, uint64_t ts,
@@ -371,69 +385,12 @@ __device__ __forceinline__ void AddTotals(unsigned long long* totals, uint64_t n
         tt += __shfl_xor(static_cast<unsigned long long>(tt), off);
         ts += __shfl_xor(static_cast<unsigned long long>(ts), off);
     }
-    if (lane == 0) {
-        atomicAdd(totals, static_cast<unsigned long long>(nt));
-        atomicAdd(totals + 1, static_cast<unsigned long long>(tt));
-        if (ts != 0) atomicAdd(totals + 2, static_cast<unsigned long long>(ts));
+    if (lane == 0 && (nt | tt | ts) != 0) {
+        unsigned long long* slot = TotalsSlot(totals);
+        atomicAdd(slot, static_cast<unsigned long long>(nt));
+        atomicAdd(slot + 1, static_cast<unsigned long long>(tt));
+        if (ts != 0) atomicAdd(slot + 2, static_cast<unsigned long long>(ts));
     }
-}
-
-// Ray claiming split into kParts ranges of the claim order, one counter each
-// (kPartStride words apart, so no two share a cache line). Workgroups are
-// dispatched to the 8 XCDs round-robin, so workgroup b starts on range
-// b % kParts: each XCD works through its own contiguous stretch of the
-// (origin-sorted) rays and its L2 keeps the nodes those rays share. A wave
-// whose range runs out moves on to the next range, so every ray is taken.
-constexpr int kParts = 8;
-constexpr int kPartStride = 32;
-
-__device__ __forceinline__ int64_t PartBegin(int part, int32_t n) {
-    return static_cast<int64_t>(part) * n / kParts;
-}
-
-__device__ __forceinline__ int32_t ClaimRayParts(uint32_t* counters, int& part_state, bool want, int lane, int32_t n,
-                                                 bool& exhausted) {
-    int part = part_state & 0xFF;
-    int parts_left = part_state >> 8;
-    uint64_t mask = Ballot(want);
-    int32_t result = -1;
-    while (mask != 0 && parts_left > 0) {
-        const int64_t lo = PartBegin(part, n);
-        const int64_t size = PartBegin(part + 1, n) - lo;
-        const int leader = __ffsll(static_cast<long long>(mask)) - 1;
-        uint32_t base = 0;
-        if (lane == leader) base = atomicAdd(counters + part * kPartStride, static_cast<uint32_t>(__popcll(mask)));
-        base = __shfl(base, leader);
-        if ((mask >> lane) & 1ull) {
-            const uint64_t mine = static_cast<uint64_t>(base) + static_cast<uint64_t>(__popcll(mask & LanesBelow(lane)));
-            if (mine < static_cast<uint64_t>(size)) result = static_cast<int32_t>(lo + static_cast<int64_t>(mine));
-        }
-        mask = Ballot(want && result < 0);
-        if (mask != 0) {  // this range is used up
-            part = part + 1 == kParts ? 0 : part + 1;
-            --parts_left;
-        }
-    }
-    part_state = part | (parts_left << 8);
-    if (want && result < 0) exhausted = true;
-    return result;
-}
-
-// Claims one ray index per wanting lane with a single atomic per wave.
-__device__ __forceinline__ int32_t ClaimRay(uint32_t* counter, bool want, int lane, int32_t n, bool& exhausted) {
-    const uint64_t mask = Ballot(want);
-    if (mask == 0) return -1;
-    const int leader = __ffsll(static_cast<long long>(mask)) - 1;
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(counter, static_cast<uint32_t>(__popcll(mask)));
-    base = __shfl(base, leader);
-    if (!want) return -1;
-    const uint32_t mine = base + static_cast<uint32_t>(__popcll(mask & LanesBelow(lane)));
-    if (mine >= static_cast<uint32_t>(n)) {
-        exhausted = true;
-        return -1;
-    }
-    return static_cast<int32_t>(mine);
 }
 
 __device__ __forceinline__ void TransformRay(const float4& r0, const float4& r1, const float4& r2, float ox, float oy,
@@ -471,36 +428,106 @@ struct RayArrayPolicy {
     }
 };
 
-// Rays a wave works through: claiming, the per-launch test sums, and the idle
-// lanes at which the wave stops traversing to refill.
+// Rays a wave works through. The claim order is split into kParts contiguous
+// stretches; workgroups are dispatched to the 8 XCDs round-robin and workgroup
+// b takes part in stretch b % kParts, so each XCD works through rays that lie
+// together and its L2 keeps the nodes they share.
+//
+// A queue with at most 64 rays per wave is dealt out by position: no atomic,
+// and the rays lie on spread_waves waves (two per SIMD) if they can, so a small
+// queue runs at the latency of few lanes per wave (4096 rays on 20 k triangles:
+// 139 us in full waves, 105, 96, 91 and 90 us on 1, 2, 4 and 8 waves per SIMD;
+// the short bounces of a Cornell frame pay for the extra waves, 2.14, 2.14,
+// 2.23 and 2.69 ms; 8 instanced cameras 48.2, 46.2, 45.4, 47.2 ms). A longer one keeps a counter per stretch; a wave claims
+// as many rays as it has idle lanes with one atomic and moves on to the next
+// stretch when its own is used up. (Dealing the first 64 by position there too
+// cost 1.29 M instanced rays 569 -> 606 us, and reading the counters before
+// moving on cost 8.39 M rays 4.1 -> 4.8 ms.)
 struct RaySource {
-    int part_state;  // claim range (low byte) and ranges left to try (next byte), wave-uniform
-    bool exhausted;
+    int part;          // the stretch this wave claims from
+    int parts_left;    // stretches not yet found used up (0: dealt by position)
+    int32_t pos, end;  // claimed rays that no lane has yet (claim positions)
+    bool drained;      // no rays left to claim
     uint32_t sum_nt, sum_tt, sum_ts;  // this lane's test counts since its last flush
 
-    __device__ __forceinline__ void Init() {
-        part_state = static_cast<int>(blockIdx.x % kParts) | (kParts << 8);
-        exhausted = false;
+    // Waves that n rays keep busy: 4 rays per lane, or spread thinner if that
+    // leaves SIMDs without a wave.
+    static __host__ __device__ __forceinline__ int32_t Waves(int64_t n, int32_t spread_waves) {
+        const int64_t full = (n + 255) / 256, spread = n < spread_waves ? n : spread_waves;
+        return static_cast<int32_t>(full > spread ? full : spread);
+    }
+    // False: this workgroup has nothing to do (a queue shorter than its grid
+    // was sized for).
+    __device__ __forceinline__ bool Init(const TraceArgs& a, int32_t n) {
+        const int32_t waves_per_group = static_cast<int32_t>(blockDim.x >> 6);
+        int32_t groups = (Waves(n, a.spread_waves) + waves_per_group - 1) / waves_per_group;
+        if (groups > static_cast<int32_t>(gridDim.x)) groups = static_cast<int32_t>(gridDim.x);
+        if (static_cast<int32_t>(blockIdx.x) >= groups) return false;
+        const int32_t waves = groups * waves_per_group;
+        const int32_t lanes = (n - 1) / waves + 1;
+        part = static_cast<int>(blockIdx.x % kParts);
+        parts_left = lanes > 64 ? kParts : 0;
+        pos = end = 0;
+        if (lanes <= 64) {
+            const int32_t extra = groups % kParts;
+            const int32_t group = part * (groups / kParts) + (part < extra ? part : extra) +
+                                  static_cast<int32_t>(blockIdx.x / kParts);
+            const int32_t wave = __builtin_amdgcn_readfirstlane(group * waves_per_group +
+                                                                static_cast<int32_t>(threadIdx.x >> 6));
+            pos = wave * lanes < n ? wave * lanes : n;
+            end = pos + lanes < n ? pos + lanes : n;
+        }
+        drained = false;
         sum_nt = sum_tt = sum_ts = 0;
+        return true;
+    }
+    // Claims up to `need` rays; false: none are left.
+    __device__ __forceinline__ bool NextRays(const TraceArgs& a, int32_t need, int lane, int32_t n) {
+        while (parts_left > 0) {
+            const int32_t lo = static_cast<int32_t>(static_cast<int64_t>(part) * n / kParts);
+            const int32_t hi = static_cast<int32_t>(static_cast<int64_t>(part + 1) * n / kParts);
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(a.counter + part * kPartStride, static_cast<uint32_t>(need));
+            base = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(base)));
+            if (base < static_cast<uint32_t>(hi - lo)) {
+                pos = lo + static_cast<int32_t>(base);
+                end = hi - pos > need ? pos + need : hi;
+                return true;
+            }
+            part = part + 1 == kParts ? 0 : part + 1;
+            --parts_left;
+        }
+        return false;
     }
     __device__ __forceinline__ void Count(const TraceArgs& a, uint32_t nt, uint32_t tt, uint32_t ts) {
         sum_nt += nt;
         sum_tt += tt;
         sum_ts += ts;
         if (a.totals != nullptr && (sum_nt | sum_tt | sum_ts) >= 0x80000000u) {  // keep 32-bit sums from wrapping
-            atomicAdd(a.totals, static_cast<unsigned long long>(sum_nt));
-            atomicAdd(a.totals + 1, static_cast<unsigned long long>(sum_tt));
-            atomicAdd(a.totals + 2, static_cast<unsigned long long>(sum_ts));
+            unsigned long long* slot = TotalsSlot(a.totals);
+            atomicAdd(slot, static_cast<unsigned long long>(sum_nt));
+            atomicAdd(slot + 1, static_cast<unsigned long long>(sum_tt));
+            atomicAdd(slot + 2, static_cast<unsigned long long>(sum_ts));
             sum_nt = sum_tt = sum_ts = 0;
         }
     }
     // The ray index a lane without one gets, or -1.
     __device__ __forceinline__ int32_t Claim(const TraceArgs& a, int32_t ray, int lane, int32_t n) {
-        const bool want = ray < 0 && !exhausted;
-        const int32_t claimed = a.parts > 1 ? ClaimRayParts(a.counter, part_state, want, lane, n, exhausted)
-                                            : ClaimRay(a.counter, want, lane, n, exhausted);
-        if (claimed < 0) return -1;
-        if (a.order != nullptr) {
+        uint64_t mask = Ballot(ray < 0);
+        int32_t claimed = -1;
+        while (mask != 0 && !drained) {
+            const int32_t need = static_cast<int32_t>(__popcll(mask));
+            if (pos == end && !NextRays(a, need, lane, n)) {
+                drained = true;
+                break;
+            }
+            const int32_t rank = static_cast<int32_t>(__popcll(mask & LanesBelow(lane)));
+            const int32_t avail = end - pos;
+            if (((mask >> lane) & 1ull) && rank < avail) claimed = pos + rank;
+            pos += need < avail ? need : avail;
+            mask = Ballot(ray < 0 && claimed < 0);
+        }
+        if (claimed >= 0 && a.order != nullptr) {
             const int32_t mapped = a.order[claimed];
             if (static_cast<uint32_t>(mapped) < static_cast<uint32_t>(n)) return mapped;
         }
@@ -509,8 +536,8 @@ struct RaySource {
 };
 
 __device__ __forceinline__ void ZeroNextCounters(const TraceArgs& a) {
-    if (a.next_counter != nullptr && blockIdx.x == 0 && threadIdx.x < static_cast<unsigned>(a.parts)) {
-        a.next_counter[threadIdx.x * (a.parts > 1 ? kPartStride : 1)] = 0u;
+    if (a.next_counter != nullptr && blockIdx.x == 0 && threadIdx.x < kParts) {
+        a.next_counter[threadIdx.x * kPartStride] = 0u;
     }
 }
 
@@ -524,7 +551,7 @@ __device__ __forceinline__ void TraceFlatLoop(const TraceArgs& a, const Policy& 
     ZeroNextCounters(a);
     const int32_t n = a.n_device != nullptr ? static_cast<int32_t>(*a.n_device) : a.n;
     RaySource src;
-    src.Init();
+    if (!src.Init(a, n)) return;
     int32_t ray = -1;
     float dx = 0, dy = 0, dz = 0, t_min = 0;
     RayPre pre{};
@@ -571,7 +598,7 @@ __device__ __forceinline__ void TraceFlatLoop(const TraceArgs& a, const Policy& 
         }
         // Lanes that hold a ray, or could still get one: when enough of them
         // are idle, the wave comes back here.
-        const uint64_t wanted = Ballot(ray >= 0 || !src.exhausted);
+        const uint64_t wanted = Ballot(ray >= 0 || !src.drained);
         if (wanted == 0) break;
 
         while (true) {
@@ -621,7 +648,7 @@ __device__ __forceinline__ void TraceTwoLevelLoop(const TraceArgs& a, const Poli
     ZeroNextCounters(a);
     const int32_t n = a.n_device != nullptr ? static_cast<int32_t>(*a.n_device) : a.n;
     RaySource src;
-    src.Init();
+    if (!src.Init(a, n)) return;
     int32_t ray = -1;
     float ox = 0, oy = 0, oz = 0, dx = 0, dy = 0, dz = 0, t_min = 0;  // the world ray
     // The ray being traversed: the world ray in the TLAS, the object ray inside
@@ -685,7 +712,7 @@ __device__ __forceinline__ void TraceTwoLevelLoop(const TraceArgs& a, const Poli
             pol.Begin(ray, o4, d4);
             start(o4, d4);
         }
-        const uint64_t wanted = Ballot(ray >= 0 || !src.exhausted);
+        const uint64_t wanted = Ballot(ray >= 0 || !src.drained);
         if (wanted == 0) break;
 
         while (true) {
