@@ -31,6 +31,10 @@ namespace yrh {
 namespace {
 
 constexpr int kBlock = 256;
+// Shade's workgroup: one queue append per 512 paths. Atomics on the append
+// word pass at one per 14 ns, so two per 256 paths took 0.45 ms of a 4.2 M-path
+// bounce, all of Shade's time.
+constexpr int kShadeBlock = 512;
 constexpr int kMaxTransparentShadowHits = 16;  // src/integrators/path_direct_lighting.cpp:19
 constexpr int kMaxAlphaSkips = 64;              // src/integrators/surface_query.cpp:12
 constexpr float kAlphaSkipOffset = 1.0e-4f;     // surface_query.cpp:13
@@ -39,19 +43,34 @@ constexpr int kHasNormals = 1;
 constexpr int kHasUvs = 2;
 constexpr int kHasTangents = 4;
 
-// Counter words of one pass (uint32).
+// Counter words of one pass (uint32): a header, then a ring of kRing bounce
+// slots. Slot d % kRing holds what bounce d consumes and claims. Three slots
+// are enough to leave clearing to the kernels that run anyway: Shade d appends
+// to slot d + 1 and clears slot d + 2, whose last users (bounce d - 1's shadow
+// rays and Resolve) have ended by then; Raygen clears the whole ring.
 enum Counter : int {
-    kCountQueue0 = 0,
-    kCountQueue1 = 1,
-    kCountShadow = 2,
-    kCountPassPaths = 3,  // paths of the current pass (batched passes)
-    kPassIndex = 4,       // current pass of a batch schedule (advanced by EndPassKernel)
-    // Per-launch ray counters of the trace kernels: one per claim range
-    // (trav::kParts ranges, trav::kPartStride words apart).
+    kCountPassPaths = 0,  // paths of the current pass (batched passes)
+    kPassIndex = 1,       // current pass of a batch schedule (advanced by EndPassKernel)
+    kHeaderWords = 32,
+};
+constexpr int kRing = 3;
+// Words of a slot.
+enum BounceWord : int {
+    // Path segments queued for bounce d and, right after them, the shadow
+    // rays of bounce d - 1: Shade appends to both with one 64-bit atomic.
+    kCountQueue = 0,
+    kCountShadow = 1,
+    // Per-launch ray counters of bounce d's traversals (trav::kParts ranges,
+    // trav::kPartStride words apart).
     kWorkExtend = 32,
     kWorkShadow = kWorkExtend + trav::kParts * trav::kPartStride,
-    kCounterWords = kWorkShadow + trav::kParts * trav::kPartStride,
+    kSlotWords = kWorkShadow + trav::kParts * trav::kPartStride,
 };
+constexpr int kCounterWords = kHeaderWords + kRing * kSlotWords;
+
+__host__ __device__ inline uint32_t* BounceSlot(uint32_t* counters, int depth) {
+    return counters + kHeaderWords + (depth % kRing) * kSlotWords;
+}
 
 // 64-bit statistics words.
 enum Stat : int {
@@ -361,6 +380,34 @@ __device__ __forceinline__ int32_t BlockAppend(uint32_t* counter, uint32_t count
     for (int w = 0; w < wave; ++w) base += lds[w];
     __syncthreads();  // lds is reused by the next call
     return count != 0u ? static_cast<int32_t>(base + inc - count) : -1;
+}
+
+// Appends `next` (0..1) entries to one queue and `shadow` (0..3) to another per
+// thread, their counts in the low and high half of *counters (all threads
+// must call; `lds`: kShadeBlock / 64 + 1 words). Returns this thread's first
+// slots in .x and .y (meaningful where it appends).
+__device__ __forceinline__ int2 AppendPair(unsigned long long* counters, uint32_t next, uint32_t shadow,
+                                           unsigned long long* lds) {
+    constexpr int kWaves = kShadeBlock / 64;
+    const int lane = Lane();
+    const int wave = static_cast<int>(threadIdx.x >> 6);
+    uint32_t inc = next | (shadow << 16);  // inclusive prefixes over the wave (at most 64 and 192)
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t up = __shfl_up(inc, off);
+        if (lane >= off) inc += up;
+    }
+    if (lane == 63) lds[wave] = (inc & 0xFFFFu) | (static_cast<unsigned long long>(inc >> 16) << 32);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long total = 0;
+        for (int w = 0; w < kWaves; ++w) total += lds[w];
+        lds[kWaves] = total != 0u ? atomicAdd(counters, total) : 0u;
+    }
+    __syncthreads();
+    unsigned long long base = lds[kWaves];
+    for (int w = 0; w < wave; ++w) base += lds[w];
+    return make_int2(static_cast<int32_t>(static_cast<uint32_t>(base) + (inc & 0xFFFFu) - next),
+                     static_cast<int32_t>(static_cast<uint32_t>(base >> 32) + (inc >> 16) - shadow));
 }
 
 // Wave-summed statistics word `word`, one atomic per wave into this
@@ -742,6 +789,12 @@ __device__ __forceinline__ AnalyticSample SampleAnalytic(const LightView& L, flo
 
 __global__ void RaygenKernel(PassView P) {
     const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    uint32_t* queued = BounceSlot(P.counters, 0);
+    if (blockIdx.x == 0) {  // path 0's thread writes the first bounce's count
+        for (int k = kHeaderWords + static_cast<int>(threadIdx.x); k < kCounterWords; k += static_cast<int>(blockDim.x)) {
+            if (P.counters + k != queued + kCountQueue) P.counters[k] = 0u;
+        }
+    }
     int64_t pixel;
     int x, y, sample, spp, width, height;
     DevCamera camera;
@@ -752,7 +805,7 @@ __global__ void RaygenKernel(PassView P) {
         const DevItem last = P.items[ie - 1];
         const int64_t total = last.path_begin + last.pixel_count;
         if (p == 0) {
-            P.counters[kCountQueue0] = static_cast<uint32_t>(total);
+            queued[kCountQueue] = static_cast<uint32_t>(total);
             P.counters[kCountPassPaths] = static_cast<uint32_t>(total);
         }
         if (p >= total) return;
@@ -784,7 +837,7 @@ __global__ void RaygenKernel(PassView P) {
         // paths e, e + n, e + 2n, ... (n listed pixels).
         const int64_t n = *P.active_count;
         const int64_t total = n * P.sample_count;
-        if (p == 0) P.counters[kCountQueue0] = static_cast<uint32_t>(total);
+        if (p == 0) queued[kCountQueue] = static_cast<uint32_t>(total);
         if (p >= total) return;
         pixel = P.active_list[p % n];
         x = static_cast<int>(pixel % P.width);
@@ -797,7 +850,7 @@ __global__ void RaygenKernel(PassView P) {
         camera = P.camera;
     } else {
         const int64_t total = P.npix * P.sample_count;
-        if (p == 0) P.counters[kCountQueue0] = static_cast<uint32_t>(total);
+        if (p == 0) queued[kCountQueue] = static_cast<uint32_t>(total);
         if (p >= total) return;
         pixel = p % P.npix;
         x = static_cast<int>(pixel % P.width);
@@ -833,24 +886,6 @@ __global__ void RaygenKernel(PassView P) {
     P.p_alb[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     P.p_nrm[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     P.p_slot[p] = make_int4(-1, -1, -1, -1);
-}
-
-// Zeroes the counters a bounce appends to before anything uses them.
-// Zeroes the counters a bounce uses before anything uses them: kBeginTrace
-// the path-segment claim counters (before the bounce's traversal), kBeginShade
-// the next queue's count, the shadow queue's count and its claim counters
-// (before Shade appends to them).
-constexpr int kBeginTrace = 1;
-constexpr int kBeginShade = 2;
-
-__global__ void BeginBounceKernel(uint32_t* counters, int next_queue, int what) {
-    const int i = static_cast<int>(threadIdx.x);
-    if (what & kBeginShade) {
-        if (i == 0) counters[next_queue] = 0u;
-        if (i == 1) counters[kCountShadow] = 0u;
-        if (i >= 2 && i < 2 + trav::kParts) counters[kWorkShadow + (i - 2) * trav::kPartStride] = 0u;
-    }
-    if ((what & kBeginTrace) && i < trav::kParts) counters[kWorkExtend + i * trav::kPartStride] = 0u;
 }
 
 struct SurfacePoint {
@@ -1341,10 +1376,15 @@ __device__ __forceinline__ void ShadePath(const PassView& P, const SurfaceView& 
 }
 
 template <bool kGuided, bool kAnalytic, bool kTex>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void ShadeKernel(PassView P, SurfaceView S, LightView L, yrg::GuideView G,
+__global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(4))) void ShadeKernel(PassView P, SurfaceView S, LightView L, yrg::GuideView G,
                                                      int depth, int cur) {
     const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    const int n = static_cast<int>(P.counters[cur]);
+    const int n = static_cast<int>(BounceSlot(P.counters, depth)[kCountQueue]);
+    if (blockIdx.x == 0) {
+        uint32_t* later = BounceSlot(P.counters, depth + 2);
+        for (int k = static_cast<int>(threadIdx.x); k < kSlotWords; k += kShadeBlock) later[k] = 0u;
+    }
+    if (static_cast<int>(blockIdx.x * blockDim.x) >= n) return;
     ShadeOut o;
     o.next = false;
     o.shadow[kShadowEmissive] = o.shadow[kShadowAnalytic] = o.shadow[kShadowEnv] = false;
@@ -1352,18 +1392,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const bool valid = i < n;
     if (valid) ShadePath<kGuided, kAnalytic, kTex>(P, S, L, G, depth, i, cur, o, hit_count, miss_count);
     const int nxt = 1 - cur;
-    __shared__ uint32_t append_lds[kBlock / 64 + 1];
-    const int32_t slot = BlockAppend(P.counters + nxt, o.next ? 1u : 0u, append_lds);
-    if (slot >= 0) {
-        const int p = P.q_path[cur][i];
-        P.q_org[nxt][slot] = F4(o.next_org, 1.0e-5f);
-        P.q_dir[nxt][slot] = F4(o.next_dir, __int_as_float(0x7f800000));
-        P.q_path[nxt][slot] = p;
-    }
-    int slot_of[kShadowKinds] = {-1, -1, -1};
     uint32_t wanted = 0;
     for (int k = 0; k < kShadowKinds; ++k) wanted += (k != kShadowAnalytic || kAnalytic) && o.shadow[k] ? 1u : 0u;
-    int32_t s = BlockAppend(P.counters + kCountShadow, wanted, append_lds);
+    __shared__ unsigned long long append_lds[kShadeBlock / 64 + 1];
+    const int2 slot = AppendPair(reinterpret_cast<unsigned long long*>(BounceSlot(P.counters, depth + 1)),
+                                 o.next ? 1u : 0u, wanted, append_lds);
+    if (o.next) {
+        const int p = P.q_path[cur][i];
+        P.q_org[nxt][slot.x] = F4(o.next_org, 1.0e-5f);
+        P.q_dir[nxt][slot.x] = F4(o.next_dir, __int_as_float(0x7f800000));
+        P.q_path[nxt][slot.x] = p;
+    }
+    int slot_of[kShadowKinds] = {-1, -1, -1};
+    int32_t s = slot.y;
     for (int k = 0; k < kShadowKinds; ++k) {
         if ((k != kShadowAnalytic || kAnalytic) && o.shadow[k]) {
             P.s_org[s] = F4(o.s_org[k], 1.0e-5f);
@@ -1405,13 +1446,13 @@ constexpr int kQueryWaves = kQueryBlock / 64;
 
 template <bool kTex>
 __global__ __launch_bounds__(kQueryBlock) void GuideQueryKernel(PassView P, SurfaceView S, LightView L,
-                                                               yrg::GuideView G, int cur) {
+                                                               yrg::GuideView G, int depth, int cur) {
     // Per wave, first the inputs of its 64 rows (stride 11: odd, no bank
     // conflicts), then the network outputs of 16 rows at a time.
     __shared__ float lds_stage[kQueryWaves][16 * yrg::kOutStride];
     static_assert(16 * yrg::kOutStride >= 64 * 11, "staging area holds the inputs");
     __shared__ yrg::bf16x8_t lds_w[yrg::kFwdFragCount * 64];  // forward weight fragments, shared by the block
-    const int n = static_cast<int>(P.counters[cur]);
+    const int n = static_cast<int>(BounceSlot(P.counters, depth)[kCountQueue]);
     if (static_cast<int64_t>(blockIdx.x) * blockDim.x >= n) return;  // whole block idle
     for (int k = static_cast<int>(threadIdx.x); k < yrg::kFwdFragCount * 64; k += kQueryBlock) lds_w[k] = G.frag[k];
     const int lane = static_cast<int>(threadIdx.x & 63u);
@@ -1561,7 +1602,7 @@ __global__ __launch_bounds__(kBlock) void GuideCollectKernel(PassView P, yrg::Gu
 // analytic, then environment, as EstimateDirectLight sums them.
 __global__ __launch_bounds__(kBlock) void ResolveKernel(PassView P, yrg::GuideView G, int depth, int cur) {
     const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    const int n = static_cast<int>(P.counters[cur]);
+    const int n = static_cast<int>(BounceSlot(P.counters, depth)[kCountQueue]);
     unsigned shadow = 0, occluded = 0;
     if (i < n) {
         const int p = P.q_path[cur][i];
@@ -1845,10 +1886,10 @@ template <bool kGuided, bool kAnalytic>
 void LaunchShade(bool textured, int grid, hipStream_t st, const PassView& P, const SurfaceView& S, const LightView& L,
                  const yrg::GuideView& G, int depth, int cur) {
     if (textured) {
-        hipLaunchKernelGGL((ShadeKernel<kGuided, kAnalytic, true>), dim3(grid), dim3(kBlock), 0, st, P, S, L, G, depth,
+        hipLaunchKernelGGL((ShadeKernel<kGuided, kAnalytic, true>), dim3(grid), dim3(kShadeBlock), 0, st, P, S, L, G, depth,
                            cur);
     } else {
-        hipLaunchKernelGGL((ShadeKernel<kGuided, kAnalytic, false>), dim3(grid), dim3(kBlock), 0, st, P, S, L, G, depth,
+        hipLaunchKernelGGL((ShadeKernel<kGuided, kAnalytic, false>), dim3(grid), dim3(kShadeBlock), 0, st, P, S, L, G, depth,
                            cur);
     }
 }
@@ -2270,15 +2311,14 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
     for (int depth = 0; depth < max_depth; ++depth) {
         const StageRange bounce_range("bounce");
         const int cur = depth & 1;
-        hipLaunchKernelGGL(BeginBounceKernel, dim3(1), dim3(64), 0, st, P.counters, 1 - cur, kBeginTrace);
         TraceRequest tr;
         tr.any = false;
         tr.org = P.q_org[cur];
         tr.dir = P.q_dir[cur];
-        tr.n_device = P.counters + cur;
+        tr.n_device = BounceSlot(P.counters, depth) + kCountQueue;
         tr.capacity = paths;
         tr.expected = paths;
-        tr.work_counter = P.counters + kWorkExtend;
+        tr.work_counter = BounceSlot(P.counters, depth) + kWorkExtend;
         tr.hit = P.hits;
         tr.instance = ctx->geo.accel_kind == YRH_ACCEL_TWO_LEVEL ? P.hit_inst : nullptr;
         tr.totals = P.stats + kStatNodeTests;
@@ -2303,20 +2343,19 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
         if (guide_here) {
             if (textured) {
                 hipLaunchKernelGGL(GuideQueryKernel<true>, dim3(Grid(paths, kQueryBlock)), dim3(kQueryBlock), 0, st, Pk,
-                                   S, L, GV, cur);
+                                   S, L, GV, depth, cur);
             } else {
                 hipLaunchKernelGGL(GuideQueryKernel<false>, dim3(Grid(paths, kQueryBlock)), dim3(kQueryBlock), 0, st, Pk,
-                                   S, L, GV, cur);
+                                   S, L, GV, depth, cur);
             }
         }
-        // The previous bounce's Resolve reads this bounce's path queue count,
-        // the path slots and the shadow queue, which Shade rewrites.
+        // The previous bounce's Resolve reads the path slots and the shadow
+        // queue, which Shade rewrites, and the counter slot that it clears.
         if (overlap && depth > 0 && (rc = CheckHip(ctx, hipStreamWaitEvent(st, resolved, 0), "hipStreamWaitEvent")) != YRH_OK) {
             return rc;
         }
-        hipLaunchKernelGGL(BeginBounceKernel, dim3(1), dim3(64), 0, st, P.counters, 1 - cur, kBeginShade);
         const bool analytic = L.analytic_count > 0;
-        const int sgrid = Grid(paths);
+        const int sgrid = Grid(paths, kShadeBlock);
         if (guide_here) {
             if (analytic) {
                 LaunchShade<true, true>(textured, sgrid, st, Pk, S, L, GV, depth, cur);
@@ -2337,10 +2376,10 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
             sr.any = true;
             sr.org = P.s_org;
             sr.dir = P.s_dir;
-            sr.n_device = P.counters + kCountShadow;
+            sr.n_device = BounceSlot(P.counters, depth + 1) + kCountShadow;
             sr.capacity = R.shadow_slots * paths;
             sr.expected = paths;  // about one shadow ray per path in flight
-            sr.work_counter = P.counters + kWorkShadow;
+            sr.work_counter = BounceSlot(P.counters, depth) + kWorkShadow;
                 sr.occluded = P.s_occ;
             sr.totals = P.stats + kStatNodeTests;
             sr.aux = overlap;
@@ -2350,10 +2389,10 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
             wr.any = false;
             wr.org = P.s_org;
             wr.dir = P.s_dir;
-            wr.n_device = P.counters + kCountShadow;
+            wr.n_device = BounceSlot(P.counters, depth + 1) + kCountShadow;
             wr.capacity = R.shadow_slots * paths;
             wr.expected = paths;
-            wr.work_counter = P.counters + kWorkShadow;
+            wr.work_counter = BounceSlot(P.counters, depth) + kWorkShadow;
                 wr.hit = P.s_trans;  // not written by the walk; LaunchTrace's checks want an output
             wr.totals = P.stats + kStatNodeTests;
             wr.aux = overlap;
@@ -3112,7 +3151,7 @@ int yrh_batch_render(yrh_context* ctx, const yrh_batch_desc* d, float* job_ms, i
         TraceRequest warm;
         warm.org = P.s_org;
         warm.dir = P.s_dir;
-        warm.n_device = P.counters + kCountShadow;
+        warm.n_device = BounceSlot(P.counters, 1) + kCountShadow;
         warm.capacity = R.shadow_slots * capacity;
         trav::TraceArgs wa;
         int g = 0, b = 0;
