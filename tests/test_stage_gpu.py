@@ -1,0 +1,33 @@
+"""Large host copies go through pinned buffers on several threads: every byte
+arrives, in both directions, at sizes around the chunk and thread limits."""
+import numpy as np
+import pytest
+
+from yaoray_amd import Device
+from yaoray_amd.api import DeviceBuffer
+
+pytestmark = pytest.mark.gpu
+
+MIB = 1 << 20
+
+
+@pytest.mark.parametrize("nbytes", [2 * MIB - 1, 2 * MIB, 2 * MIB + 1, 3 * MIB, 5 * MIB + 4093, 16 * MIB, 17 * MIB + 1,
+                                    32 * MIB, 41 * MIB + 7])
+def test_large_copies_arrive_whole(nbytes):
+    rng = np.random.default_rng(nbytes)
+    dev = Device(0)  # its first copy is plain unless it is very large
+    try:
+        buf = DeviceBuffer(dev, nbytes + 64)
+        guard = np.full(64, 7, np.uint8)
+        for _ in range(3):
+            a = rng.integers(0, 256, nbytes, np.uint8)
+            buf.upload(np.concatenate([np.zeros(nbytes, np.uint8), guard]))
+            buf.upload(a)
+            out = np.full(nbytes + 64, 3, np.uint8)
+            dev._check(dev._lib.yrh_copy_to_host(dev._ctx, out.ctypes.data, buf.ptr, nbytes), "copy_to_host")
+            assert np.array_equal(out[:nbytes], a)
+            assert (out[nbytes:] == 3).all()
+            assert np.array_equal(buf.download(np.uint8, nbytes + 64)[nbytes:], guard)
+        buf.free()
+    finally:
+        dev.close()

@@ -334,6 +334,7 @@ void yrh_destroy(yrh_context* ctx) {
     if (ctx->aux_stream != nullptr) (void)hipStreamSynchronize(ctx->aux_stream);
     DestroyRenderState(ctx);
     DestroyGuideState(ctx);
+    DestroyHostStage(ctx);
     ctx->geo = DevGeometry{};
     ctx->work_counter.reset();
     ctx->stack_spill.reset();
@@ -387,7 +388,10 @@ int yrh_device_free(yrh_context* ctx, void* ptr) {
 int yrh_copy_to_device(yrh_context* ctx, void* dst, const void* src, size_t bytes) {
     if (ctx == nullptr || (bytes > 0 && (dst == nullptr || src == nullptr))) return YRH_E_INVALID_ARGUMENT;
     if (bytes == 0) return YRH_OK;
-    int rc = CheckHip(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream), "hipMemcpyAsync H2D");
+    bool done = false;
+    int rc = StagedCopyToDevice(ctx, dst, src, bytes, &done);
+    if (done || rc != YRH_OK) return rc;
+    rc = CheckHip(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream), "hipMemcpyAsync H2D");
     if (rc != YRH_OK) return rc;
     return CheckHip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
 }
@@ -395,7 +399,10 @@ int yrh_copy_to_device(yrh_context* ctx, void* dst, const void* src, size_t byte
 int yrh_copy_to_host(yrh_context* ctx, void* dst, const void* src, size_t bytes) {
     if (ctx == nullptr || (bytes > 0 && (dst == nullptr || src == nullptr))) return YRH_E_INVALID_ARGUMENT;
     if (bytes == 0) return YRH_OK;
-    int rc = CheckHip(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync D2H");
+    bool done = false;
+    int rc = StagedCopyToHost(ctx, dst, src, bytes, &done);
+    if (done || rc != YRH_OK) return rc;
+    rc = CheckHip(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync D2H");
     if (rc != YRH_OK) return rc;
     return CheckHip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
 }

@@ -1,0 +1,172 @@
+// Large copies between pageable host memory and the device.
+//
+// What bounds them: a plain hipMemcpyAsync on pageable memory is staged by the
+// runtime 1 MiB at a time on one thread, which also takes the page faults of a
+// freshly allocated destination: 12 GB/s for a film read, against about 50
+// GB/s of the link. Here a few threads copy chunks through pinned buffers of
+// the context: while one chunk is on the link, the same thread moves the one
+// before it to or from the caller's memory.
+#include "yrh_internal.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+namespace yrh {
+
+namespace {
+
+constexpr size_t kChunk = size_t{1} << 20;
+constexpr int kMaxThreads = 8;  // the caller's among them
+constexpr int kSlots = 2 * kMaxThreads;
+// Below, starting threads costs what the copy gains (4 MiB: 45 us slower).
+constexpr size_t kMinBytes = size_t{6} << 20;
+// Chunks per thread that pay for starting one.
+constexpr size_t kChunksPerThread = 2;
+
+}  // namespace
+
+struct HostStage {
+    char* memory = nullptr;  // kSlots chunks, pinned
+    hipEvent_t events[kSlots] = {};
+    ~HostStage() {
+        for (hipEvent_t e : events) {
+            if (e != nullptr) (void)hipEventDestroy(e);
+        }
+        if (memory != nullptr) (void)hipHostFree(memory);
+    }
+};
+
+void DestroyHostStage(yrh_context* ctx) {
+    delete ctx->stage;
+    ctx->stage = nullptr;
+}
+
+namespace {
+
+// The context's pinned buffers (16 MiB), or null: copies too small to gain,
+// a context's first copy unless it pays for the allocation by itself (a
+// context made for one frame reads one film), or no pinned memory to be had.
+HostStage* Stage(yrh_context* ctx, size_t bytes) {
+    if (bytes < kMinBytes) return nullptr;
+    if (ctx->stage != nullptr) return ctx->stage;
+    if (!ctx->large_copy_seen && bytes < (size_t{32} << 20)) {
+        ctx->large_copy_seen = true;
+        return nullptr;
+    }
+    HostStage* s = new HostStage();
+    bool ok = hipHostMalloc(reinterpret_cast<void**>(&s->memory), kSlots * kChunk, hipHostMallocDefault) == hipSuccess;
+    for (int k = 0; ok && k < kSlots; ++k) {
+        ok = hipEventCreateWithFlags(&s->events[k], hipEventDisableTiming) == hipSuccess;
+    }
+    if (!ok) {
+        (void)hipGetLastError();
+        delete s;
+        return nullptr;
+    }
+    ctx->stage = s;
+    return s;
+}
+
+// Runs `work(k)` on as many threads as the copy fills, the caller's included.
+template <class Work>
+void RunThreads(size_t chunks, const Work& work) {
+    const int threads = static_cast<int>(
+        std::max<size_t>(1, std::min<size_t>(kMaxThreads, chunks / kChunksPerThread)));
+    std::vector<std::thread> pool;
+    try {
+        pool.reserve(static_cast<size_t>(threads));
+        for (int k = 1; k < threads; ++k) pool.emplace_back(work, k);
+    } catch (const std::system_error&) {  // no more threads: the ones there take all chunks
+    }
+    work(0);
+    for (std::thread& t : pool) t.join();
+}
+
+}  // namespace
+
+int StagedCopyToHost(yrh_context* ctx, void* dst, const void* src, size_t bytes, bool* done) {
+    HostStage* s = Stage(ctx, bytes);
+    *done = s != nullptr;
+    if (s == nullptr) return YRH_OK;
+    const size_t chunks = (bytes + kChunk - 1) / kChunk;
+    std::atomic<size_t> next{0};
+    std::atomic<int> status{hipSuccess};
+    auto work = [&](int thread) {
+        (void)hipSetDevice(ctx->device);
+        size_t held[2] = {chunks, chunks};  // the chunk in each of the thread's slots (chunks: none)
+        for (int turn = 0;; turn ^= 1) {
+            const int slot = 2 * thread + turn;
+            const size_t c = status.load() == hipSuccess ? next.fetch_add(1) : chunks;
+            held[turn] = c < chunks ? c : chunks;
+            if (c < chunks) {
+                const size_t at = c * kChunk;
+                hipError_t e = hipMemcpyAsync(s->memory + static_cast<size_t>(slot) * kChunk,
+                                              static_cast<const char*>(src) + at, std::min(kChunk, bytes - at),
+                                              hipMemcpyDeviceToHost, ctx->stream);
+                if (e == hipSuccess) e = hipEventRecord(s->events[slot], ctx->stream);
+                if (e != hipSuccess) {
+                    status.store(e);
+                    held[turn] = chunks;
+                }
+            }
+            // The chunk before it, meanwhile.
+            const int other = turn ^ 1;
+            if (held[other] < chunks) {
+                const int oslot = 2 * thread + other;
+                const hipError_t e = hipEventSynchronize(s->events[oslot]);
+                if (e != hipSuccess) {
+                    status.store(e);
+                } else {
+                    const size_t at = held[other] * kChunk;
+                    std::memcpy(static_cast<char*>(dst) + at, s->memory + static_cast<size_t>(oslot) * kChunk,
+                                std::min(kChunk, bytes - at));
+                }
+                held[other] = chunks;
+            } else if (held[turn] == chunks) {
+                return;
+            }
+        }
+    };
+    RunThreads(chunks, work);
+    const hipError_t sync = hipStreamSynchronize(ctx->stream);
+    const hipError_t e = static_cast<hipError_t>(status.load());
+    return CheckHip(ctx, e != hipSuccess ? e : sync, "staged copy to host");
+}
+
+int StagedCopyToDevice(yrh_context* ctx, void* dst, const void* src, size_t bytes, bool* done) {
+    HostStage* s = Stage(ctx, bytes);
+    *done = s != nullptr;
+    if (s == nullptr) return YRH_OK;
+    const size_t chunks = (bytes + kChunk - 1) / kChunk;
+    std::atomic<size_t> next{0};
+    std::atomic<int> status{hipSuccess};
+    auto work = [&](int thread) {
+        (void)hipSetDevice(ctx->device);
+        bool used[2] = {false, false};
+        for (int turn = 0;; turn ^= 1) {
+            const int slot = 2 * thread + turn;
+            const size_t c = status.load() == hipSuccess ? next.fetch_add(1) : chunks;
+            if (c >= chunks) return;
+            const size_t at = c * kChunk, n = std::min(kChunk, bytes - at);
+            char* pinned = s->memory + static_cast<size_t>(slot) * kChunk;
+            hipError_t e = used[turn] ? hipEventSynchronize(s->events[slot]) : hipSuccess;
+            if (e == hipSuccess) {
+                std::memcpy(pinned, static_cast<const char*>(src) + at, n);
+                e = hipMemcpyAsync(static_cast<char*>(dst) + at, pinned, n, hipMemcpyHostToDevice, ctx->stream);
+            }
+            if (e == hipSuccess) e = hipEventRecord(s->events[slot], ctx->stream);
+            if (e != hipSuccess) status.store(e);
+            used[turn] = true;
+        }
+    };
+    RunThreads(chunks, work);
+    const hipError_t sync = hipStreamSynchronize(ctx->stream);
+    const hipError_t e = static_cast<hipError_t>(status.load());
+    return CheckHip(ctx, e != hipSuccess ? e : sync, "staged copy to device");
+}
+
+}  // namespace yrh
