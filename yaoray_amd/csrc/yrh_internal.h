@@ -158,7 +158,7 @@ struct yrh_context {
     // own spill region. Default priority, like the main stream.
     hipStream_t aux_stream = nullptr;
     yrh::DevBuf stack_spill_aux;
-    hipEvent_t bounce_events[2] = {nullptr, nullptr};  // [0] shaded, [1] shadows resolved
+    hipEvent_t bounce_events[3] = {};  // [0] shaded, [1..2] shadows of even / odd bounces resolved
     bool render_overlap = true;
     // Launch shape of the persistent traversal kernels; 0 = chosen per launch
     // (yrh_trace.hip PrepareTraceArgs: 8 LDS stack levels and 8 workgroups per

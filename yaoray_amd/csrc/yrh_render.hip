@@ -44,16 +44,17 @@ constexpr int kHasUvs = 2;
 constexpr int kHasTangents = 4;
 
 // Counter words of one pass (uint32): a header, then a ring of kRing bounce
-// slots. Slot d % kRing holds what bounce d consumes and claims. Three slots
-// are enough to leave clearing to the kernels that run anyway: Shade d appends
-// to slot d + 1 and clears slot d + 2, whose last users (bounce d - 1's shadow
-// rays and Resolve) have ended by then; Raygen clears the whole ring.
+// slots. Slot d % kRing holds what bounce d consumes and claims. Clearing is
+// left to kernels that run anyway: Shade d appends to slot d + 1 and clears
+// slot d + 2, which bounce d - 2's shadow rays and Resolve, ended by then, were
+// the last to use (bounce d - 1's, which may still run, use slots d - 1 and d);
+// Raygen clears the whole ring.
 enum Counter : int {
     kCountPassPaths = 0,  // paths of the current pass (batched passes)
     kPassIndex = 1,       // current pass of a batch schedule (advanced by EndPassKernel)
     kHeaderWords = 32,
 };
-constexpr int kRing = 3;
+constexpr int kRing = 4;
 // Words of a slot.
 enum BounceWord : int {
     // Path segments queued for bounce d and, right after them, the shadow
@@ -96,6 +97,13 @@ static_assert(kStatSlots == trav::kTotalsSlots && kStatStride == trav::kTotalsSt
 constexpr size_t kStatBytes = sizeof(unsigned long long) * kStatStride * kStatSlots;
 
 }  // namespace
+
+// An array within RenderState::pass.
+struct Slice {
+    void* ptr = nullptr;
+    template <typename T>
+    T* as() const { return static_cast<T*>(ptr); }
+};
 
 struct RenderState {
     // ---- surface geometry (shading copy) ----
@@ -151,8 +159,8 @@ struct RenderState {
     int32_t analytic_tree_count = 0;
     int32_t analytic_tree_root = -1;
     int32_t use_analytic_tree = 0;
-    // Shadow-queue entries per path slot: emissive, analytic (scenes with
-    // analytic lights), environment.
+    // Shadow-queue entries per path slot: one for each kind of light that the
+    // scene has (emissive, analytic, a sampled environment).
     int shadow_slots = 2;
     int cap_shadow_slots = 0;
     // environment
@@ -183,16 +191,23 @@ struct RenderState {
     yrh_adaptive_desc act_desc{};
     // ---- pass buffers (capacity = paths per pass) ----
     int64_t capacity = 0;
-    DevBuf p_pixel, p_tp, p_rad, p_prev, p_flags, p_med, p_alb, p_nrm, p_nee, p_slot;  // p_slot: int4 shadow entries
+    // p_rad: emission and environment reached by the path; p_dir: its
+    // next-event contributions (the sample is their sum).
+    DevBuf pass;  // all of the arrays below, in one allocation (each hipFree takes 0.2 ms)
+    Slice p_pixel, p_tp, p_rad, p_dir, p_prev, p_flags, p_med, p_alb, p_nrm;
     DevBuf p_diff;  // float4[2] per path: the camera ray's differential directions (footprints only)
-    DevBuf q_org[2], q_dir[2], q_path[2];
-    DevBuf hits, hit_inst;
-    DevBuf s_org, s_dir, s_li, s_bsdf, s_occ, s_trans;
-    DevBuf l_state, l_med;
-    DevBuf counters;  // uint32[kCounterWords]
+    Slice q_org[2], q_dir[2], q_path[2];
+    Slice hits, hit_inst;
+    // Shadow queues of alternate bounces, and the state of the queue that is
+    // being traced (s_trans, l_*: scenes with transparent shadows).
+    Slice s_org[2], s_dir[2], s_li[2], s_bsdf[2], s_nee[2], s_occ, s_trans;
+    Slice l_state, l_med;
+    bool cap_transparent = false;
+    bool two_shadow_queues = false;
+    Slice counters;   // uint32[kCounterWords]
     DevBuf stats;     // uint64[kStatStride * kStatSlots]: kStatSlots copies of the statistics words
     // batched passes
-    DevBuf p_job, p_sample;
+    Slice p_job, p_sample;
     DevBuf b_jobs, b_items, b_pass_items, b_film;
     std::vector<int64_t> b_job_pixels;  // per job: pixel count
     std::vector<int64_t> b_job_offset;  // per job: first pixel in b_film
@@ -310,13 +325,12 @@ struct PassView {
     int32_t* p_pixel;
     float4* p_tp;
     float4* p_rad;
+    float4* p_dir;
     float4* p_prev;
     int32_t* p_flags;
     float4* p_med;
     float4* p_alb;
     float4* p_nrm;
-    float4* p_nee;
-    int4* p_slot;  // shadow-queue entries of the path's vertex: emissive, analytic, environment
     float4* p_diff;  // camera-ray differential directions (2 per path), or nullptr
     // queues
     float4* q_org[2];
@@ -324,13 +338,17 @@ struct PassView {
     int32_t* q_path[2];
     float4* hits;
     int32_t* hit_inst;
+    // Shadow queue of the bounce. A vertex's entries are consecutive, emissive,
+    // analytic, environment; the first holds their number and the path (s_bsdf.w
+    // bits: count << 30 | path, 0 in the others) and the throughput (s_nee).
     float4* s_org;
     float4* s_dir;
     float4* s_li;
     float4* s_bsdf;
+    float4* s_nee;
     uint32_t* s_occ;
-    float4* s_trans;
-    int4* l_state;
+    float4* s_trans;  // transmittance, or nullptr (opaque scenes)
+    int32_t* l_state;
     float4* l_med;
     uint32_t* counters;
     unsigned long long* stats;
@@ -885,7 +903,7 @@ __global__ void RaygenKernel(PassView P) {
     P.p_med[p] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
     P.p_alb[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     P.p_nrm[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    P.p_slot[p] = make_int4(-1, -1, -1, -1);
+    P.p_dir[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
 struct SurfacePoint {
@@ -1110,6 +1128,7 @@ struct ShadeOut {
     float s_tmax[kShadowKinds];
     float3 s_li[kShadowKinds], s_bsdf[kShadowKinds];
     float s_scale[kShadowKinds];
+    float3 nee;  // throughput arriving at the vertex
 };
 
 // ---- guided sampling (learned proposal, yrh_guide.h) ----------------------------
@@ -1168,7 +1187,6 @@ __device__ __forceinline__ void ShadePath(const PassView& P, const SurfaceView& 
     float3 tp = XYZ(P.p_tp[p]);
     float3 rad = XYZ(P.p_rad[p]);
     const float4 prev = P.p_prev[p];
-    P.p_slot[p] = make_int4(-1, -1, -1, -1);
     const int pix = P.p_pixel[p];
     PixelSampler smp;
     if (P.jobs != nullptr) {
@@ -1235,7 +1253,7 @@ __device__ __forceinline__ void ShadePath(const PassView& P, const SurfaceView& 
     // Next-event estimation (path_direct_lighting.cpp:115-283): the emissive and
     // environment samples share the DirectLightSurface 2D sample.
     if (!IsDelta(mat)) {
-        P.p_nee[p] = F4(tp, 0.0f);
+        o.nee = tp;
         const float2 surf = smp.Get2D(kDimLightSurface);
         if (L.emissive_count > 0) {
             const LightSample ls = SampleEmissive(S, L, smp.Get1D(kDimLightSelect), surf);
@@ -1362,7 +1380,7 @@ __device__ __forceinline__ void ShadePath(const PassView& P, const SurfaceView& 
             // known once the path ends (GuideCollectKernel).
             float4* r = G.rec + 4 * (static_cast<int64_t>(depth) * G.rec_paths + p);
             r[0] = F4(hp, beta_lum);
-            r[1] = F4(sn, Lum(rad));
+            r[1] = F4(sn, Lum(Add(rad, XYZ(P.p_dir[p]))));
             r[2] = F4(wo, __int_as_float(G.stamp));
             r[3] = F4(bs.wi, 0.0f);
         }
@@ -1403,21 +1421,20 @@ __global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(4))
         P.q_dir[nxt][slot.x] = F4(o.next_dir, __int_as_float(0x7f800000));
         P.q_path[nxt][slot.x] = p;
     }
-    int slot_of[kShadowKinds] = {-1, -1, -1};
     int32_t s = slot.y;
     for (int k = 0; k < kShadowKinds; ++k) {
         if ((k != kShadowAnalytic || kAnalytic) && o.shadow[k]) {
+            uint32_t owner = 0;
+            if (s == slot.y) {
+                owner = (wanted << 30) | static_cast<uint32_t>(P.q_path[cur][i]);
+                P.s_nee[s] = F4(o.nee, 0.0f);
+            }
             P.s_org[s] = F4(o.s_org[k], 1.0e-5f);
             P.s_dir[s] = F4(o.s_dir[k], o.s_tmax[k]);
             P.s_li[s] = F4(o.s_li[k], o.s_scale[k]);
-            P.s_bsdf[s] = F4(o.s_bsdf[k], 0.0f);
-            P.s_trans[s] = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
-            slot_of[k] = s;
+            P.s_bsdf[s] = F4(o.s_bsdf[k], __uint_as_float(owner));
             ++s;
         }
-    }
-    if (valid && wanted > 0) {
-        P.p_slot[P.q_path[cur][i]] = make_int4(slot_of[kShadowEmissive], slot_of[kShadowAnalytic], slot_of[kShadowEnv], -1);
     }
     WaveStat(P.stats, kStatHits, hit_count);
     WaveStat(P.stats, kStatMisses, miss_count);
@@ -1565,7 +1582,7 @@ __global__ __launch_bounds__(kBlock) void GuideCollectKernel(PassView P, yrg::Gu
         if (slot < total) {
             const float4* r = G.rec + 4 * slot;
             if (__float_as_int(r[2].w) == G.stamp) {
-                const float final_lum = Lum(XYZ(P.p_rad[slot % G.rec_paths]));
+                const float final_lum = Lum(Add(XYZ(P.p_rad[slot % G.rec_paths]), XYZ(P.p_dir[slot % G.rec_paths])));
                 w[j] = (final_lum - r[1].w) / r[0].w;
                 if (isfinite(w[j]) && w[j] > 0.0f) keep |= 1u << j;
             }
@@ -1599,37 +1616,42 @@ __global__ __launch_bounds__(kBlock) void GuideCollectKernel(PassView P, yrg::Gu
 }
 
 // Adds the visible next-event contributions of this bounce, emissive, then
-// analytic, then environment, as EstimateDirectLight sums them.
-__global__ __launch_bounds__(kBlock) void ResolveKernel(PassView P, yrg::GuideView G, int depth, int cur) {
-    const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    const int n = static_cast<int>(BounceSlot(P.counters, depth)[kCountQueue]);
+// analytic, then environment, as EstimateDirectLight sums them. They go to a
+// sum of their own, so Shade never waits for the shadow rays of the bounce
+// before. A fixed grid walks the shadow queue (a thread per path slot, most of
+// them past the end of a late bounce's queue, took 120 us a bounce on 33 M
+// paths).
+constexpr int kResolveGroupsPerCu = 8;
+
+__global__ __launch_bounds__(kBlock) void ResolveKernel(PassView P, yrg::GuideView G, int depth) {
+    const int n = static_cast<int>(BounceSlot(P.counters, depth + 1)[kCountShadow]);
     unsigned shadow = 0, occluded = 0;
-    if (i < n) {
-        const int p = P.q_path[cur][i];
-        const int4 slots = P.p_slot[p];
-        if (slots.x >= 0 || slots.y >= 0 || slots.z >= 0) {
-            float3 direct = V(0.0f, 0.0f, 0.0f);
-            for (int k = 0; k < kShadowKinds; ++k) {
-                const int s = k == kShadowEmissive ? slots.x : (k == kShadowAnalytic ? slots.y : slots.z);
-                if (s < 0) continue;
-                ++shadow;
-                if (P.s_occ[s] != 0u) {
-                    ++occluded;
-                    continue;
-                }
-                const float4 li = P.s_li[s];
-                const float3 c = Mul(Hadamard(XYZ(P.s_bsdf[s]), Hadamard(XYZ(P.s_trans[s]), XYZ(li))), li.w);
-                direct = Add(direct, c);
+    for (int64_t e = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; e < n;
+         e += static_cast<int64_t>(gridDim.x) * kBlock) {
+        const float4 b0 = P.s_bsdf[e];
+        const uint32_t owner = __float_as_uint(b0.w);
+        const int count = static_cast<int>(owner >> 30);
+        if (count == 0) continue;
+        const int p = static_cast<int>(owner & 0x3FFFFFFFu);
+        float3 direct = V(0.0f, 0.0f, 0.0f);
+        for (int k = 0; k < count; ++k) {
+            ++shadow;
+            if (P.s_occ[e + k] != 0u) {
+                ++occluded;
+                continue;
             }
-            const float3 tp = XYZ(P.p_nee[p]);
-            const float3 rad = Add(XYZ(P.p_rad[p]), Hadamard(tp, direct));
-            P.p_rad[p] = F4(rad, 0.0f);
-            if (G.rec != nullptr) {
-                // This vertex's own next-event estimate is not radiance along
-                // its sampled direction: move the record's snapshot past it.
-                float4* r = G.rec + 4 * (static_cast<int64_t>(depth) * G.rec_paths + p);
-                if (__float_as_int(r[2].w) == G.stamp) r[1].w = Lum(rad);
-            }
+            const float4 li = P.s_li[e + k];
+            const float3 bsdf = k == 0 ? XYZ(b0) : XYZ(P.s_bsdf[e + k]);
+            const float3 seen = P.s_trans != nullptr ? Hadamard(XYZ(P.s_trans[e + k]), XYZ(li)) : XYZ(li);
+            direct = Add(direct, Mul(Hadamard(bsdf, seen), li.w));
+        }
+        const float3 sum = Add(XYZ(P.p_dir[p]), Hadamard(XYZ(P.s_nee[e]), direct));
+        P.p_dir[p] = F4(sum, 0.0f);
+        if (G.rec != nullptr) {
+            // This vertex's own next-event estimate is not radiance along
+            // its sampled direction: move the record's snapshot past it.
+            float4* r = G.rec + 4 * (static_cast<int64_t>(depth) * G.rec_paths + p);
+            if (__float_as_int(r[2].w) == G.stamp) r[1].w = Lum(Add(XYZ(P.p_rad[p]), sum));
         }
     }
     WaveStat(P.stats, kStatShadow, shadow);
@@ -1640,11 +1662,14 @@ __global__ __launch_bounds__(kBlock) void ResolveKernel(PassView P, yrg::GuideVi
 // One persistent launch walks every shadow ray through its dielectric surfaces:
 // the traversal hands each closest hit to ShadowWalk::Finish, which applies the
 // reference's per-hit rule and returns the next segment (same lane) until the
-// ray is decided. l_state[e] = (0, transparent hits so far, finite, 0);
+// ray is decided. l_state[e]: transparent hits so far (low byte), kWalkFinite,
+// alpha skips of the segment (high half);
 // l_med[e] = medium (color, distance; distance < 0 = inactive); s_trans holds
 // the transmittance and the remaining distance in .w.
 
 __device__ __forceinline__ bool TransBlack(float3 c) { return MaxC(c) <= 1.0e-6f; }
+
+constexpr int32_t kWalkFinite = 0x100;
 
 template <bool kAlpha, bool kTex>
 struct ShadowWalk {
@@ -1655,7 +1680,7 @@ struct ShadowWalk {
     __device__ __forceinline__ void Begin(int32_t e, float4& o, float4& d) const {
         o = P->s_org[e];
         d = P->s_dir[e];
-        P->l_state[e] = make_int4(0, 0, isfinite(d.w) ? 1 : 0, 0);
+        P->l_state[e] = isfinite(d.w) ? kWalkFinite : 0;
         P->l_med[e] = make_float4(1.0f, 1.0f, 1.0f, -1.0f);
         P->s_trans[e] = make_float4(1.0f, 1.0f, 1.0f, d.w);
     }
@@ -1663,12 +1688,14 @@ struct ShadowWalk {
     __device__ __forceinline__ bool Finish(int32_t e, const trav::Best& best, int32_t inst, uint32_t, uint32_t,
                                            uint32_t, const float4& lo, const float4& ld, float4& next_org,
                                            float4& next_dir) const {
-        int4 st = P->l_state[e];
+        const int32_t state = P->l_state[e];
+        int hits = state & 0xFF, skips = state >> 16;
         const float4 tr = P->s_trans[e];
         float3 T = XYZ(tr);
         float remaining = tr.w;
         float4 med = P->l_med[e];
-        const bool finite = st.z != 0;
+        const bool finite = (state & kWalkFinite) != 0;
+        auto packed = [&]() { return hits | (state & kWalkFinite) | (skips << 16); };
         uint32_t occ = 1u;
         bool again = false;
         bool hit = best.Hit();
@@ -1679,15 +1706,15 @@ struct ShadowWalk {
             // hit; past the segment's end it is a miss, and the 64th skipped
             // hit leaves the segment exhausted, which blocks the shadow ray.
             const float t_min = best.t + kAlphaSkipOffset;
-            st.w += 1;
+            ++skips;
             if (t_min >= remaining) {
                 hit = false;
-            } else if (st.w >= kMaxAlphaSkips) {
+            } else if (skips >= kMaxAlphaSkips) {
                 P->s_occ[e] = 1u;
-                P->l_state[e] = st;
+                P->l_state[e] = packed();
                 return false;
             } else {
-                P->l_state[e] = st;
+                P->l_state[e] = packed();
                 next_org = make_float4(lo.x, lo.y, lo.z, t_min);
                 next_dir = make_float4(ld.x, ld.y, ld.z, remaining);
                 return true;
@@ -1749,12 +1776,12 @@ struct ShadowWalk {
                     }
                 }
                 if (!done) {
-                    st.y += 1;
-                    if (st.y >= kMaxTransparentShadowHits) {
+                    ++hits;
+                    if (hits >= kMaxTransparentShadowHits) {
                         occ = 1u;
                     } else {
                         again = true;
-                        st.w = 0;  // a new segment: its own alpha skips
+                        skips = 0;  // a new segment: its own alpha skips
                         next_org = F4(Add(hp, Mul(XYZ(ld), bias)), 1.0e-5f);
                         next_dir = make_float4(ld.x, ld.y, ld.z, remaining);
                     }
@@ -1764,7 +1791,7 @@ struct ShadowWalk {
         P->s_occ[e] = occ;
         P->s_trans[e] = F4(T, remaining);
         P->l_med[e] = med;
-        P->l_state[e] = st;
+        P->l_state[e] = packed();
         return again;
     }
 };
@@ -1899,7 +1926,7 @@ void LaunchShade(bool textured, int grid, hipStream_t st, const PassView& P, con
 __device__ __forceinline__ unsigned AddSample(const PassView& P, int64_t p, yrh_film_pixel& px) {
     unsigned bad = 0;
     {
-        float3 b = XYZ(P.p_rad[p]);
+        float3 b = Add(XYZ(P.p_rad[p]), XYZ(P.p_dir[p]));
         if (P.radiance_clamp > 0.0f) {
             const float m = MaxC(b);
             if (!(m <= P.radiance_clamp || m <= 0.0f)) b = Mul(b, P.radiance_clamp / m);
@@ -2049,6 +2076,16 @@ __global__ void SampleValuesKernel(int kind, uint64_t seed, int spp, int64_t n, 
 
 int Grid(int64_t n, int block = kBlock) { return static_cast<int>(std::max<int64_t>(1, (n + block - 1) / block)); }
 
+// The shadow queue of bounce `depth`.
+void SetShadowQueue(const RenderState& R, PassView& P, int depth) {
+    const int k = R.two_shadow_queues ? depth & 1 : 0;
+    P.s_org = R.s_org[k].as<float4>();
+    P.s_dir = R.s_dir[k].as<float4>();
+    P.s_li = R.s_li[k].as<float4>();
+    P.s_bsdf = R.s_bsdf[k].as<float4>();
+    P.s_nee = R.s_nee[k].as<float4>();
+}
+
 PassView MakePassView(RenderState& R, const yrh_render_desc& d) {
     PassView P{};
     P.width = d.width;
@@ -2069,13 +2106,12 @@ PassView MakePassView(RenderState& R, const yrh_render_desc& d) {
     P.p_pixel = R.p_pixel.as<int32_t>();
     P.p_tp = R.p_tp.as<float4>();
     P.p_rad = R.p_rad.as<float4>();
+    P.p_dir = R.p_dir.as<float4>();
     P.p_prev = R.p_prev.as<float4>();
     P.p_flags = R.p_flags.as<int32_t>();
     P.p_med = R.p_med.as<float4>();
     P.p_alb = R.p_alb.as<float4>();
     P.p_nrm = R.p_nrm.as<float4>();
-    P.p_nee = R.p_nee.as<float4>();
-    P.p_slot = R.p_slot.as<int4>();
     P.p_diff = R.footprints ? R.p_diff.as<float4>() : nullptr;
     for (int k = 0; k < 2; ++k) {
         P.q_org[k] = R.q_org[k].as<float4>();
@@ -2084,13 +2120,10 @@ PassView MakePassView(RenderState& R, const yrh_render_desc& d) {
     }
     P.hits = R.hits.as<float4>();
     P.hit_inst = R.hit_inst.as<int32_t>();
-    P.s_org = R.s_org.as<float4>();
-    P.s_dir = R.s_dir.as<float4>();
-    P.s_li = R.s_li.as<float4>();
-    P.s_bsdf = R.s_bsdf.as<float4>();
+    SetShadowQueue(R, P, 0);
     P.s_occ = R.s_occ.as<uint32_t>();
-    P.s_trans = R.s_trans.as<float4>();
-    P.l_state = R.l_state.as<int4>();
+    P.s_trans = R.transparent ? R.s_trans.as<float4>() : nullptr;
+    P.l_state = R.l_state.as<int32_t>();
     P.l_med = R.l_med.as<float4>();
     P.counters = R.counters.as<uint32_t>();
     P.stats = R.stats.as<unsigned long long>();
@@ -2227,8 +2260,9 @@ __global__ void BsdfQueryKernel(const DevMaterial* mats, int64_t n, const int32_
 
 // Bytes per path slot and per shadow slot of the arrays EnsureCapacity
 // allocates, and per guided row (mixture + valid flag).
-constexpr size_t kPathSlotBytes = 4 + 4 + 4 + 16 + 16 + 16 + 4 + 16 + 16 + 16 + 16 + 16 + 2 * 16 + 2 * 16 + 2 * 4 + 16 + 4;
-constexpr size_t kShadowSlotBytes = 16 + 16 + 16 + 16 + 4 + 16 + 16 + 16;
+constexpr size_t kPathSlotBytes = 4 + 4 + 4 + 16 + 16 + 16 + 16 + 4 + 16 + 16 + 16 + 2 * 16 + 2 * 16 + 2 * 4 + 16 + 4;
+constexpr size_t kShadowSlotBytes = 2 * 5 * 16 + 4;
+constexpr size_t kWalkSlotBytes = 16 + 4 + 16;  // transparent shadows only
 constexpr size_t kGuideRowBytes = yrg::kGuideMixtureRow * 4 + 4;
 
 // The camera-ray differentials (two float4 per path) of scenes whose textures
@@ -2240,8 +2274,14 @@ int EnsureDifferentials(yrh_context* ctx, RenderState& R) {
     return rc != YRH_OK ? rc : Alloc(ctx, R.p_diff, bytes);
 }
 
+// Allocates the pass buffers for `paths` path slots, in one block: 30 of their
+// own cost a context made for one frame 7 ms to free. Two shadow queues for
+// alternate bounces, or one (each Shade then waits for the Resolve before it)
+// without overlap, or where the second would take more than a quarter of the
+// memory left (the film, the guide's rows and the stack spill still need some).
 int EnsureCapacity(yrh_context* ctx, RenderState& R, int64_t paths) {
-    if (R.capacity >= paths && R.cap_shadow_slots >= R.shadow_slots && R.counters.ptr != nullptr) {
+    if (R.capacity >= paths && R.cap_shadow_slots >= R.shadow_slots && (R.cap_transparent || !R.transparent) &&
+        R.counters.ptr != nullptr) {
         return EnsureDifferentials(ctx, R);
     }
     int rc = CheckHip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
@@ -2249,20 +2289,38 @@ int EnsureCapacity(yrh_context* ctx, RenderState& R, int64_t paths) {
     paths = std::max(paths, R.capacity);
     const size_t P = static_cast<size_t>(paths);
     const size_t S = static_cast<size_t>(R.shadow_slots) * P;
+    const size_t W = R.transparent ? S : 1;  // transparent walks
     struct Item {
-        DevBuf* buf;
+        Slice* slice;
         size_t bytes;
     } items[] = {
+        {&R.counters, 4 * kCounterWords},
         {&R.p_pixel, 4 * P}, {&R.p_job, 4 * P}, {&R.p_sample, 4 * P}, {&R.p_tp, 16 * P}, {&R.p_rad, 16 * P}, {&R.p_prev, 16 * P}, {&R.p_flags, 4 * P},
-        {&R.p_med, 16 * P}, {&R.p_alb, 16 * P}, {&R.p_nrm, 16 * P}, {&R.p_nee, 16 * P}, {&R.p_slot, 16 * P},
+        {&R.p_med, 16 * P}, {&R.p_alb, 16 * P}, {&R.p_nrm, 16 * P}, {&R.p_dir, 16 * P},
         {&R.q_org[0], 16 * P}, {&R.q_org[1], 16 * P}, {&R.q_dir[0], 16 * P}, {&R.q_dir[1], 16 * P},
         {&R.q_path[0], 4 * P}, {&R.q_path[1], 4 * P}, {&R.hits, 16 * P}, {&R.hit_inst, 4 * P},
-        {&R.s_org, 16 * S}, {&R.s_dir, 16 * S}, {&R.s_li, 16 * S}, {&R.s_bsdf, 16 * S}, {&R.s_occ, 4 * S},
-        {&R.s_trans, 16 * S}, {&R.l_state, 16 * S}, {&R.l_med, 16 * S},
-        {&R.counters, 4 * kCounterWords},
+        {&R.s_occ, 4 * S}, {&R.s_trans, 16 * W}, {&R.l_state, 4 * W}, {&R.l_med, 16 * W},
+        {&R.s_org[0], 16 * S}, {&R.s_dir[0], 16 * S}, {&R.s_li[0], 16 * S}, {&R.s_bsdf[0], 16 * S}, {&R.s_nee[0], 16 * S},
+        {&R.s_org[1], 16 * S}, {&R.s_dir[1], 16 * S}, {&R.s_li[1], 16 * S}, {&R.s_bsdf[1], 16 * S}, {&R.s_nee[1], 16 * S},
     };
-    for (const Item& it : items) {
-        if ((rc = Alloc(ctx, *it.buf, it.bytes)) != YRH_OK) return rc;
+    constexpr size_t kSecondQueue = 5;  // the last items
+    auto padded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    size_t total = 0, second = 0;
+    for (size_t k = 0; k < std::size(items); ++k) {
+        (k + kSecondQueue < std::size(items) ? total : second) += padded(items[k].bytes);
+    }
+    R.capacity = 0;
+    R.pass.reset();
+    size_t free_bytes = 0, device_bytes = 0;
+    if ((rc = CheckHip(ctx, hipMemGetInfo(&free_bytes, &device_bytes), "hipMemGetInfo")) != YRH_OK) return rc;
+    R.two_shadow_queues = ctx->render_overlap && free_bytes >= total && free_bytes - total >= 4 * second;
+    if (R.two_shadow_queues) total += second;
+    if ((rc = Alloc(ctx, R.pass, total)) != YRH_OK) return rc;
+    char* at = R.pass.as<char>();
+    for (size_t k = 0; k < std::size(items); ++k) {
+        const bool held = R.two_shadow_queues || k + kSecondQueue < std::size(items);
+        items[k].slice->ptr = held ? at : nullptr;
+        if (held) at += padded(items[k].bytes);
     }
     if (R.stats.ptr == nullptr) {
         if ((rc = Alloc(ctx, R.stats, kStatBytes)) != YRH_OK) return rc;
@@ -2273,7 +2331,25 @@ int EnsureCapacity(yrh_context* ctx, RenderState& R, int64_t paths) {
     rc = CheckHip(ctx, hipMemsetAsync(R.counters.ptr, 0, 4 * kCounterWords, ctx->stream), "hipMemsetAsync");
     R.capacity = paths;
     R.cap_shadow_slots = R.shadow_slots;
+    R.cap_transparent = R.transparent;
     return rc != YRH_OK ? rc : EnsureDifferentials(ctx, R);
+}
+
+// The second stream and the events of overlapped bounces.
+int EnsureOverlap(yrh_context* ctx) {
+    int rc;
+    if (ctx->aux_stream == nullptr &&
+        (rc = CheckHip(ctx, hipStreamCreateWithFlags(&ctx->aux_stream, hipStreamNonBlocking), "hipStreamCreate")) !=
+            YRH_OK) {
+        return rc;
+    }
+    for (hipEvent_t& e : ctx->bounce_events) {
+        if (e == nullptr &&
+            (rc = CheckHip(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate")) != YRH_OK) {
+            return rc;
+        }
+    }
+    return YRH_OK;
 }
 
 // Raygen and the bounces of one pass over `paths` path slots (the queue
@@ -2284,26 +2360,21 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
     const bool guided = GV.mode != YRH_GUIDE_OFF;
     int rc;
     // Overlap: a bounce's shadow rays and Resolve run on the second stream
-    // while the main stream traces the next bounce's path segments (and
-    // queries the guide); Shade of the next bounce waits for that Resolve.
-    // Every per-path operation keeps its order, so the film is the same.
+    // while the main stream goes on with the next bounce. Shade waits for the
+    // Resolve of two bounces before, whose shadow queue and counter slot it
+    // reuses (of the bounce before while vertices are recorded: the records
+    // hold the radiance so far). Every sum keeps its order, so the film is the
+    // same. A walk through glass ends with a few long rays, which stood in the
+    // way of every bounce: 8 instanced cameras 43.3 -> 34.4 ms (one stream
+    // before), Cornell frame 1.96 -> 1.88 ms, textured frame 5.65 -> 5.56 ms.
     hipStream_t ss = st;
     if (overlap) {
-        if (ctx->aux_stream == nullptr &&
-            (rc = CheckHip(ctx, hipStreamCreateWithFlags(&ctx->aux_stream, hipStreamNonBlocking), "hipStreamCreate")) !=
-                YRH_OK) {
-            return rc;
-        }
-        for (hipEvent_t& e : ctx->bounce_events) {
-            if (e == nullptr &&
-                (rc = CheckHip(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate")) != YRH_OK) {
-                return rc;
-            }
-        }
+        if ((rc = EnsureOverlap(ctx)) != YRH_OK) return rc;
         ss = ctx->aux_stream;
     }
-    hipEvent_t shaded = overlap ? ctx->bounce_events[0] : nullptr;
-    hipEvent_t resolved = overlap ? ctx->bounce_events[1] : nullptr;
+    hipEvent_t shaded = ctx->bounce_events[0];
+    hipEvent_t* resolved = ctx->bounce_events + 1;
+    const int lag = GV.rec != nullptr || !R.two_shadow_queues ? 1 : 2;
     {
         const StageRange r("raygen");
         hipLaunchKernelGGL(RaygenKernel, dim3(Grid(paths)), dim3(kBlock), 0, st, P);
@@ -2323,6 +2394,7 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
         tr.instance = ctx->geo.accel_kind == YRH_ACCEL_TWO_LEVEL ? P.hit_inst : nullptr;
         tr.totals = P.stats + kStatNodeTests;
         PassView Pk = P;
+        SetShadowQueue(R, Pk, depth);
         if (ctx->geo.accel_kind != YRH_ACCEL_TWO_LEVEL) Pk.hit_inst = nullptr;
         if (depth > 0) Pk.p_diff = nullptr;  // only camera rays carry differentials
         if (R.alpha) {
@@ -2349,9 +2421,8 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
                                    S, L, GV, depth, cur);
             }
         }
-        // The previous bounce's Resolve reads the path slots and the shadow
-        // queue, which Shade rewrites, and the counter slot that it clears.
-        if (overlap && depth > 0 && (rc = CheckHip(ctx, hipStreamWaitEvent(st, resolved, 0), "hipStreamWaitEvent")) != YRH_OK) {
+        if (overlap && depth >= lag &&
+            (rc = CheckHip(ctx, hipStreamWaitEvent(st, resolved[(depth - lag) & 1], 0), "hipStreamWaitEvent")) != YRH_OK) {
             return rc;
         }
         const bool analytic = L.analytic_count > 0;
@@ -2374,8 +2445,8 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
         if (!R.transparent) {
             TraceRequest sr;
             sr.any = true;
-            sr.org = P.s_org;
-            sr.dir = P.s_dir;
+            sr.org = Pk.s_org;
+            sr.dir = Pk.s_dir;
             sr.n_device = BounceSlot(P.counters, depth + 1) + kCountShadow;
             sr.capacity = R.shadow_slots * paths;
             sr.expected = paths;  // about one shadow ray per path in flight
@@ -2387,8 +2458,8 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
         } else {
             TraceRequest wr;
             wr.any = false;
-            wr.org = P.s_org;
-            wr.dir = P.s_dir;
+            wr.org = Pk.s_org;
+            wr.dir = Pk.s_dir;
             wr.n_device = BounceSlot(P.counters, depth + 1) + kCountShadow;
             wr.capacity = R.shadow_slots * paths;
             wr.expected = paths;
@@ -2401,16 +2472,19 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
             if ((rc = PrepareTraceArgs(ctx, wr, wa, wgrid, wblock)) != YRH_OK) return rc;
             if (ctx->geo.accel_kind == YRH_ACCEL_TWO_LEVEL) {
                 LaunchShadowWalk<true>(ctx->geo.has_spheres, R.alpha, R.textured, wgrid, wblock, LdsBytes(wa, wblock), ss,
-                                       wa, P, S, L);
+                                       wa, Pk, S, L);
             } else {
                 LaunchShadowWalk<false>(ctx->geo.has_spheres, R.alpha, R.textured, wgrid, wblock, LdsBytes(wa, wblock), ss,
-                                        wa, P, S, L);
+                                        wa, Pk, S, L);
             }
         }
-        hipLaunchKernelGGL(ResolveKernel, dim3(Grid(paths)), dim3(kBlock), 0, ss, P, GV, depth, cur);
-        if (overlap && (rc = CheckHip(ctx, hipEventRecord(resolved, ss), "hipEventRecord")) != YRH_OK) return rc;
+        hipLaunchKernelGGL(ResolveKernel, dim3(std::min(Grid(paths), kResolveGroupsPerCu * ctx->compute_units)), dim3(kBlock),
+                           0, ss, Pk, GV, depth);
+        if (overlap && (rc = CheckHip(ctx, hipEventRecord(resolved[depth & 1], ss), "hipEventRecord")) != YRH_OK) return rc;
     }
-    if (overlap && (rc = CheckHip(ctx, hipStreamWaitEvent(st, resolved, 0), "hipStreamWaitEvent")) != YRH_OK) return rc;
+    if (overlap && (rc = CheckHip(ctx, hipStreamWaitEvent(st, resolved[(max_depth - 1) & 1], 0), "hipStreamWaitEvent")) != YRH_OK) {
+        return rc;
+    }
     if ((rc = CheckHip(ctx, hipGetLastError(), "pass sequence launch")) != YRH_OK) return rc;
     if (GV.rec != nullptr) {
         hipLaunchKernelGGL(GuideCollectKernel, dim3(Grid(paths * max_depth, kBlock * kCollectPer)), dim3(kBlock), 0, st,
@@ -2813,7 +2887,6 @@ int yrh_upload_shading(yrh_context* ctx, const yrh_shading_desc* sd) {
         R.analytic_tree_count = nt;
         R.analytic_tree_root = nt > 0 ? sd->analytic_tree_root : -1;
         R.use_analytic_tree = nt > 0 ? 1 : 0;
-        R.shadow_slots = na > 0 ? 3 : 2;
     }
     // Primitive -> first emitter record (the reference's linear scan).
     {
@@ -2843,6 +2916,7 @@ int yrh_upload_shading(yrh_context* ctx, const yrh_shading_desc* sd) {
     if ((rc = UploadVec(ctx, R.env_texels, reinterpret_cast<const float4*>(env.texels), env_texels)) != YRH_OK) return rc;
     const bool has_tex = env_texels > 0;
     R.env_sampleable = (env.active && env.strength > 0.0f && has_tex && env.has_distribution) ? 1 : 0;
+    R.shadow_slots = std::max(1, (R.emissive_count > 0) + (R.analytic_count > 0) + (R.env_sampleable != 0));
     R.env_dw = env.has_distribution ? env.dist_width : 0;
     R.env_dh = env.has_distribution ? env.dist_height : 0;
     R.env_total = env.total_weight;
@@ -2989,7 +3063,9 @@ int yrh_suggest_paths_per_pass(yrh_context* ctx, int32_t max_depth, int64_t* pat
     if (rc != YRH_OK) return rc;
     // Per path: the path slot state (EnsureCapacity) and its shadow slots.
     const int shadow_slots = ctx->render != nullptr ? ctx->render->shadow_slots : 2;
-    size_t per_path = kPathSlotBytes + static_cast<size_t>(shadow_slots) * kShadowSlotBytes;
+    const bool transparent = ctx->render == nullptr || ctx->render->transparent;
+    size_t per_path = kPathSlotBytes +
+                      static_cast<size_t>(shadow_slots) * (kShadowSlotBytes + (transparent ? kWalkSlotBytes : 0));
     if (ctx->guide != nullptr) per_path += kGuideRowBytes + 64 * static_cast<size_t>(std::max(1, max_depth));
     const size_t held = ctx->render != nullptr ? static_cast<size_t>(ctx->render->capacity) * per_path : 0;
     const int64_t fit = static_cast<int64_t>((free_bytes + held) / 2 / per_path);
@@ -3156,10 +3232,15 @@ int yrh_batch_render(yrh_context* ctx, const yrh_batch_desc* d, float* job_ms, i
         trav::TraceArgs wa;
         int g = 0, b = 0;
         if ((rc = PrepareTraceArgs(ctx, warm, wa, g, b)) != YRH_OK) return rc;
+        if (ctx->render_overlap) {
+            if ((rc = EnsureOverlap(ctx)) != YRH_OK) return rc;
+            warm.aux = true;
+            if ((rc = PrepareTraceArgs(ctx, warm, wa, g, b)) != YRH_OK) return rc;
+        }
     }
     hipStream_t st = ctx->stream;
     auto launch_pass = [&]() -> int {
-        int r = LaunchPassSequence(ctx, R, P, S, L, GV, capacity, max_depth, false);
+        int r = LaunchPassSequence(ctx, R, P, S, L, GV, capacity, max_depth, ctx->render_overlap);
         if (r != YRH_OK) return r;
         for (int32_t occ = 0; occ <= max_occurrence; ++occ) {
             hipLaunchKernelGGL(AccumulateBatchKernel, dim3(Grid(capacity)), dim3(kBlock), 0, st, P, occ);
