@@ -82,6 +82,23 @@ def test_gradients_match_bf16_oracle(device):
     assert np.all(gm[10240:].reshape(64, 48)[:, 40:] == 0.0)
 
 
+@pytest.mark.parametrize("log2,rmin,rmax,rows", [(17, 40, 64, 700), (14, 2, 12, 2100), (16, 8, 256, 4100), (12, 16, 64, 16)])
+def test_gradients_with_any_number_of_copied_levels(device, log2, rmin, rmax, rows):
+    """No level, every level and some levels added through the per-workgroup
+    copies; a second call starts from cleared copies. Tolerances: bf16 products,
+    FP32 sums in another order, as in test_gradients_match_bf16_oracle."""
+    d = guide_desc(log2, rmin, rmax)
+    configure(device, d)
+    mlp, grid = guide_params(d, 5)
+    device.guide_set_params(mlp, grid)
+    smp = guide_samples(rows, 33)
+    _, og, oloss = O.guide_gradients(d, mlp, grid, smp, 0.8, bf16=True)
+    for _ in range(2):
+        _, gg, loss = device.guide_gradients(smp, 0.8)
+        assert rel_l2(gg, og) < 2e-2
+        assert abs(loss - oloss) < 1e-3 * max(1.0, abs(oloss))
+
+
 def test_mixture_eval_matches_oracle(device):
     rng = np.random.default_rng(41)
     n = 20000

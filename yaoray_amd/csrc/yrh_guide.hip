@@ -10,6 +10,8 @@
 //                         gradient (BF16) for the weight-gradient GEMM
 //   GuideWeightGradKernel dW = H^T dZ per 16x16 tile with MFMA, K = rows,
 //                         split over row chunks (FP32 partial sums)
+//   GuideFoldKernel       adds the copies of the coarse levels' gradients and
+//                         of the loss to the gradient and the loss
 //   GuideAdamMlpKernel    sum of the partials + Adam on the FP32 master weights
 //   GuideAdamGridKernel   Adam on the touched hash-grid entries
 //   GuidePackKernel       master weights -> BF16 A-operand fragments
@@ -34,6 +36,20 @@ using yrg::f32x4_t;
 // Device memory the per-cell grid copies may take (levels coarse first).
 constexpr int64_t kGuideCellBudgetDefault = static_cast<int64_t>(512) << 20;
 
+// Gradient copies of the coarse levels. Atomics on one cache line pass at one
+// per 14 ns, and a coarse level is a few lines that every row adds to (9^3
+// entries are 46): 65536 rows took 228 us for level 0, 53 and 45 us for the
+// next two, out of 585 us for the backward kernel. Workgroup b adds those and
+// the loss to copy b % kReplicas instead.
+constexpr int kReplicas = 32;
+constexpr int kReplicaHeader = 32;          // words: [0] loss, the rest unused (a cache line)
+constexpr int64_t kCoarseEntries = 1 << 15;  // entries of the levels that are copied, at most
+struct CoarseGrid {
+    int32_t levels = 0;                      // levels 0 .. levels - 1 are copied
+    int32_t begin[yrg::kGuideLevels + 1] = {};  // their first entries
+    int32_t stride = kReplicaHeader;         // words of a copy
+};
+
 struct GuideState {
     yrh_guide_desc desc{};
     yrg::GuideGrid grid{};
@@ -42,6 +58,8 @@ struct GuideState {
     DevBuf mlp, mlp_m, mlp_v;
     DevBuf frag_fwd, frag_bwd;
     DevBuf table, table_m, table_v, table_grad;
+    DevBuf replicas;  // CoarseGrid copies, zero between steps
+    CoarseGrid coarse;
     DevBuf samples;     // float4 x 4 per recorded sample: (p, w), (n, 0), (wo, 0), (wi, 0)
     DevBuf sample_hdr;  // uint32 [0] count, [1] dropped; float [2] weight sum, [3] loss
     DevBuf partial;     // FP32 [chunks][kMlpParams]
@@ -155,10 +173,11 @@ struct TrainArgs {
     const bf16x4_t* bwd;
     const float2* table;
     float* table_grad;
+    float* replicas;
+    CoarseGrid coarse;
     yrg::GuideGrid grid;
     uint16_t* act;
     uint16_t* grad;
-    float* loss;
 };
 
 __device__ __forceinline__ void StoreBlock(uint16_t* base, bf16x4_t v, int lane) {
@@ -217,6 +236,7 @@ __global__ __launch_bounds__(kBlock) void GuideBackwardKernel(TrainArgs A) {
     const int64_t rb = static_cast<int64_t>(blockIdx.x) * 4 + wave;
     const int64_t nrb = (A.rows + 15) / 16;
     const int row = lane % 16, q = lane / 16;
+    float* copy = A.replicas + static_cast<int64_t>(blockIdx.x % kReplicas) * A.coarse.stride;
     const int64_t idx = rb * 16 + row;
     const uint32_t count = min(*A.count, A.capacity);
     const bool valid = rb < nrb && idx < A.rows && count > 0;
@@ -260,11 +280,10 @@ __global__ __launch_bounds__(kBlock) void GuideBackwardKernel(TrainArgs A) {
         float loss = 0.0f;
         HeadGradient(out, wi[0], wi[1], wi[2], c, d, loss);
         for (int j = 0; j < yrg::kGuideOut; ++j) lo[row * yrg::kOutStride + j] = d[j];
-        // One atomic per wave for the loss (lanes 0..15 hold the 16 rows):
-        // every row adding to the one word serialised the whole step.
+        // One atomic per wave for the loss (lanes 0..15 hold the 16 rows).
         if (!valid) loss = 0.0f;
         for (int off = 8; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
-        if (lane == 0 && loss != 0.0f) atomicAdd(A.loss, loss);
+        if (lane == 0 && loss != 0.0f) atomicAdd(copy, loss);
     }
     __syncthreads();
     bf16x4_t dz3[3], dz2[4], dz1[4], dz0[4];
@@ -306,7 +325,9 @@ __global__ __launch_bounds__(kBlock) void GuideBackwardKernel(TrainArgs A) {
             const float ga = valid ? dx[2 * lv] : 0.0f;
             const float gb = valid ? dx[2 * lv + 1] : 0.0f;
             const yrg::GridCell cell = yrg::LocateCell(A.grid, level, p);
-            float* g = A.table_grad + static_cast<size_t>(level) * A.grid.table_size * 2;
+            float* g = level < A.coarse.levels
+                           ? copy + kReplicaHeader + 2 * A.coarse.begin[level]
+                           : A.table_grad + static_cast<size_t>(level) * A.grid.table_size * 2;
             for (int k = 0; k < 8; ++k) {
                 const float cw = yrg::CornerWeight(cell, k);
                 float va = cw * ga, vb = cw * gb;
@@ -345,6 +366,32 @@ __global__ __launch_bounds__(kBlock) void GuideBackwardKernel(TrainArgs A) {
             StoreBlock(grd + (8 + b) * 256, dz2[b], lane);
         }
         for (int b = 0; b < 3; ++b) StoreBlock(grd + (12 + b) * 256, dz3[b], lane);
+    }
+}
+
+// Adds the copies to the gradient and the loss, and clears them.
+__global__ __launch_bounds__(kBlock) void GuideFoldKernel(float* replicas, CoarseGrid C, float* table_grad,
+                                                          uint32_t table_size, float* loss) {
+    const int i = static_cast<int>(blockIdx.x * kBlock + threadIdx.x);
+    if (i >= C.stride) return;
+    float v[kReplicas];
+#pragma unroll
+    for (int r = 0; r < kReplicas; ++r) v[r] = replicas[static_cast<int64_t>(r) * C.stride + i];
+    float sum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < kReplicas; ++r) sum += v[r];
+    float* to = nullptr;
+    if (i == 0) to = loss;
+    if (i >= kReplicaHeader) {
+        const int e = (i - kReplicaHeader) / 2;
+        int level = 0;
+        while (level + 1 < C.levels && e >= C.begin[level + 1]) ++level;
+        to = table_grad + (static_cast<size_t>(level) * table_size + static_cast<size_t>(e - C.begin[level])) * 2 + (i & 1);
+    }
+    if (to != nullptr && sum != 0.0f) *to += sum;
+#pragma unroll
+    for (int r = 0; r < kReplicas; ++r) {
+        if (v[r] != 0.0f) replicas[static_cast<int64_t>(r) * C.stride + i] = 0.0f;
     }
 }
 
@@ -618,11 +665,14 @@ int BackwardPass(yrh_context* ctx, GuideState& G, const float4* samples, const u
     A.bwd = G.frag_bwd.as<bf16x4_t>();
     A.table = G.table.as<float2>();
     A.table_grad = G.table_grad.as<float>();
+    A.replicas = G.replicas.as<float>();
+    A.coarse = G.coarse;
     A.grid = G.grid;
     A.act = G.act.as<uint16_t>();
     A.grad = G.grad.as<uint16_t>();
-    A.loss = loss;
     hipLaunchKernelGGL(GuideBackwardKernel, dim3(Grid(nrb, 4)), dim3(kBlock), 0, ctx->stream, A);
+    hipLaunchKernelGGL(GuideFoldKernel, dim3(Grid(G.coarse.stride)), dim3(kBlock), 0, ctx->stream, G.replicas.as<float>(),
+                       G.coarse, G.table_grad.as<float>(), G.grid.table_size, loss);
     hipLaunchKernelGGL(GuideWeightGradKernel, dim3(Grid(kTiles * chunks, 4)), dim3(kBlock), 0, ctx->stream,
                        G.act.as<uint16_t>(), G.grad.as<uint16_t>(), nrb, chunks, G.partial.as<float>());
     return CheckHip(ctx, hipGetLastError(), "guide backward");
@@ -724,6 +774,13 @@ int yrh_guide_configure(yrh_context* ctx, const yrh_guide_desc* d) {
         g.res[l] = static_cast<int32_t>(std::floor(d->min_resolution * std::pow(ratio, l / 7.0) + 0.5));
         g.dense[l] = std::pow(static_cast<double>(g.res[l]) + 1.0, 3.0) <= static_cast<double>(g.table_size) ? 1 : 0;
     }
+    for (int l = 0; l < yrg::kGuideLevels; ++l) {
+        const int64_t side = static_cast<int64_t>(g.res[l]) + 1;
+        if (!g.dense[l] || G->coarse.begin[l] + side * side * side > kCoarseEntries) break;
+        G->coarse.begin[l + 1] = G->coarse.begin[l] + static_cast<int32_t>(side * side * side);
+        G->coarse.levels = l + 1;
+    }
+    G->coarse.stride = kReplicaHeader + (2 * G->coarse.begin[G->coarse.levels] + 31) / 32 * 32;
     for (int a = 0; a < 3; ++a) {
         g.bmin[a] = d->bounds_min[a];
         g.inv_extent[a] = 1.0f / (d->bounds_max[a] - d->bounds_min[a]);
@@ -752,13 +809,14 @@ int yrh_guide_configure(yrh_context* ctx, const yrh_guide_desc* d) {
         (rc = Alloc(ctx, G->frag_bwd, yrg::kFragCount * 64 * 8)) != YRH_OK || (rc = Alloc(ctx, G->table, tb)) != YRH_OK ||
         (rc = Alloc(ctx, G->table_m, tb)) != YRH_OK || (rc = Alloc(ctx, G->table_v, tb)) != YRH_OK ||
         (rc = Alloc(ctx, G->table_grad, tb)) != YRH_OK ||
+        (rc = Alloc(ctx, G->replicas, static_cast<size_t>(G->coarse.stride) * kReplicas * 4)) != YRH_OK ||
         (rc = Alloc(ctx, G->samples, static_cast<size_t>(std::max(1, d->sample_capacity)) * 64)) != YRH_OK ||
         (rc = Alloc(ctx, G->sample_hdr, 16)) != YRH_OK) {
         return rc;
     }
     if ((rc = yrh_copy_to_device(ctx, G->mlp.ptr, w.data(), mb)) != YRH_OK) return rc;
     if ((rc = yrh_copy_to_device(ctx, G->table.ptr, t.data(), tb)) != YRH_OK) return rc;
-    for (DevBuf* b : {&G->mlp_m, &G->mlp_v, &G->table_m, &G->table_v, &G->table_grad, &G->sample_hdr}) {
+    for (DevBuf* b : {&G->mlp_m, &G->mlp_v, &G->table_m, &G->table_v, &G->table_grad, &G->replicas, &G->sample_hdr}) {
         if ((rc = CheckHip(ctx, hipMemsetAsync(b->ptr, 0, b->bytes, ctx->stream), "hipMemsetAsync")) != YRH_OK) return rc;
     }
     if ((rc = Pack(ctx, *G)) != YRH_OK) return rc;
