@@ -98,7 +98,7 @@ constexpr size_t kStatBytes = sizeof(unsigned long long) * kStatStride * kStatSl
 
 }  // namespace
 
-// An array within RenderState::pass.
+// An array within one of RenderState::pass.
 struct Slice {
     void* ptr = nullptr;
     template <typename T>
@@ -193,7 +193,7 @@ struct RenderState {
     int64_t capacity = 0;
     // p_rad: emission and environment reached by the path; p_dir: its
     // next-event contributions (the sample is their sum).
-    DevBuf pass;  // all of the arrays below, in one allocation (each hipFree takes 0.2 ms)
+    std::vector<DevBuf> pass;  // the arrays below, small ones together
     Slice p_pixel, p_tp, p_rad, p_dir, p_prev, p_flags, p_med, p_alb, p_nrm;
     DevBuf p_diff;  // float4[2] per path: the camera ray's differential directions (footprints only)
     Slice q_org[2], q_dir[2], q_path[2];
@@ -2274,8 +2274,12 @@ int EnsureDifferentials(yrh_context* ctx, RenderState& R) {
     return rc != YRH_OK ? rc : Alloc(ctx, R.p_diff, bytes);
 }
 
-// Allocates the pass buffers for `paths` path slots, in one block: 30 of their
-// own cost a context made for one frame 7 ms to free. Two shadow queues for
+// Small pass buffers share an allocation of up to this size (freeing 30 of
+// their own costs a context made for one frame 7 ms). Not all in one: a block of
+// 1.5 GB or 256 MiB now and then takes the driver 39 ms to hand out.
+constexpr size_t kPassBlockBytes = size_t{64} << 20;
+
+// Allocates the pass buffers for `paths` path slots. Two shadow queues for
 // alternate bounces, or one (each Shade then waits for the Resolve before it)
 // without overlap, or where the second would take more than a quarter of the
 // memory left (the film, the guide's rows and the stack spill still need some).
@@ -2305,22 +2309,29 @@ int EnsureCapacity(yrh_context* ctx, RenderState& R, int64_t paths) {
     };
     constexpr size_t kSecondQueue = 5;  // the last items
     auto padded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    const size_t first_count = std::size(items) - kSecondQueue;
     size_t total = 0, second = 0;
-    for (size_t k = 0; k < std::size(items); ++k) {
-        (k + kSecondQueue < std::size(items) ? total : second) += padded(items[k].bytes);
-    }
+    for (size_t k = 0; k < std::size(items); ++k) (k < first_count ? total : second) += padded(items[k].bytes);
     R.capacity = 0;
-    R.pass.reset();
+    R.pass.clear();
     size_t free_bytes = 0, device_bytes = 0;
     if ((rc = CheckHip(ctx, hipMemGetInfo(&free_bytes, &device_bytes), "hipMemGetInfo")) != YRH_OK) return rc;
     R.two_shadow_queues = ctx->render_overlap && free_bytes >= total && free_bytes - total >= 4 * second;
-    if (R.two_shadow_queues) total += second;
-    if ((rc = Alloc(ctx, R.pass, total)) != YRH_OK) return rc;
-    char* at = R.pass.as<char>();
-    for (size_t k = 0; k < std::size(items); ++k) {
-        const bool held = R.two_shadow_queues || k + kSecondQueue < std::size(items);
-        items[k].slice->ptr = held ? at : nullptr;
-        if (held) at += padded(items[k].bytes);
+    const size_t count = R.two_shadow_queues ? std::size(items) : first_count;
+    for (size_t k = count; k < std::size(items); ++k) items[k].slice->ptr = nullptr;
+    for (size_t k = 0; k < count;) {
+        size_t end = k, bytes = 0;
+        while (end < count && (end == k || bytes + padded(items[end].bytes) <= kPassBlockBytes)) {
+            bytes += padded(items[end].bytes);
+            ++end;
+        }
+        R.pass.emplace_back();
+        if ((rc = Alloc(ctx, R.pass.back(), bytes)) != YRH_OK) return rc;
+        char* at = R.pass.back().as<char>();
+        for (; k < end; ++k) {
+            items[k].slice->ptr = at;
+            at += padded(items[k].bytes);
+        }
     }
     if (R.stats.ptr == nullptr) {
         if ((rc = Alloc(ctx, R.stats, kStatBytes)) != YRH_OK) return rc;
