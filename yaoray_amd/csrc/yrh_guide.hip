@@ -40,7 +40,7 @@ constexpr int64_t kGuideCellBudgetDefault = static_cast<int64_t>(512) << 20;
 // per 14 ns, and a coarse level is a few lines that every row adds to (9^3
 // entries are 46): 65536 rows took 228 us for level 0, 53 and 45 us for the
 // next two, out of 585 us for the backward kernel. Workgroup b adds those and
-// the loss to copy b % kReplicas instead.
+// the loss to copy b % kReplicas instead: 352 us, and 5 us for the fold.
 constexpr int kReplicas = 32;
 constexpr int kReplicaHeader = 32;          // words: [0] loss, the rest unused (a cache line)
 constexpr int64_t kCoarseEntries = 1 << 15;  // entries of the levels that are copied, at most
