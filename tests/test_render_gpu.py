@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle_py as O
-from tests.helpers import base_path_scene
+from tests.helpers import base_path_scene, cornell_materials
 from yaoray_amd import Scene
 
 pytestmark = pytest.mark.gpu
@@ -64,6 +64,29 @@ def test_depth1_cornell_bit_exact(device):
         assert gs[k] == os_[k], k
     assert np.array_equal(g["aov_samples"], o["aov_samples"])
     assert np.array_equal(g["depth_sum"].astype(np.float32), o["depth_sum"])
+
+
+@pytest.mark.parametrize("unused", [None, {"kind": 2, "ior": 1.5}, {"kind": 0, "alpha": 0.3}],
+                         ids=["opaque", "walk", "alpha"])
+def test_triangles_without_a_flat_index_block_light(device, unused):
+    """The boxes of the Cornell box with flat index -1 (in scenes whose shadow
+    rays are any-hit queries, walks through glass, walks with alpha): paths do
+    not see them, shadow rays do. Where the camera sees no box, a depth-1 film
+    is the plain scene's."""
+    s = Scene.cornell(1)
+    if unused is not None:
+        s.set_materials(cornell_materials(s) + [unused])
+    s.build_accel()
+    whole, _ = device.render(s, 64, 64, 4, max_depth=1, seed=3)
+    g, t = s.geometry_desc(), s.flat_bvh()
+    t.primitives["flat_triangle_index"][np.isin(t.primitives["mesh_primitive"], (5, 6))] = -1  # the two boxes
+    g.flat = t.desc()
+    device.upload_geometry(g)
+    device.upload_shading(s)
+    film, _ = device.render(s, 64, 64, 4, max_depth=1, seed=3, upload=False)
+    same = (film["aov_samples"] == whole["aov_samples"]) & (film["depth_sum"] == whole["depth_sum"])
+    assert 0.3 < same.mean() < 0.95
+    assert np.array_equal(film["sum"][same], whole["sum"][same])
 
 
 def test_known_answers(device):

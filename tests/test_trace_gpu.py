@@ -183,6 +183,45 @@ def test_leaves_that_share_primitives(device, kind):
     assert (r["triangle"] >= 0).any()
 
 
+@pytest.mark.parametrize("kind", ["flat", "two_level"])
+def test_hits_on_triangles_without_a_flat_index(device, kind):
+    """A caller's tree may hold triangles whose flat index is -1: they shorten
+    the ray and occlude as any other, and their hit reports id -1."""
+    import ctypes as C
+
+    from yaoray_amd import native as N
+    org, d = random_rays(20000, seed=31)
+    if kind == "flat":
+        s = Scene.triangles(3000, seed=3)
+        trees = lambda: [s.flat_bvh()]  # noqa: E731
+    else:
+        s = Scene.instanced(instances=60, subdivisions=2, variants=3, env_width=8, env_height=4, seed=6)
+        org[:, :3] = org[:, :3] * (40.0, 6.0, 40.0) - (20.0, 1.0, 20.0)
+        trees = lambda: [s.blas(k) for k in range(s.info.blas_count)]  # noqa: E731
+    s.build_accel()
+    v, i, p = s.geometry()
+    g, trees = s.geometry_desc(), trees()
+    for t in trees:
+        t.primitives["flat_triangle_index"][::2] = -1
+    if kind == "flat":
+        g.flat = trees[0].desc()
+        oracle = lambda **k: O.trace_flat(v, i, p, trees[0], org, d, **k)  # noqa: E731
+    else:
+        blases = (N.BvhDesc * len(trees))(*[t.desc() for t in trees])
+        g.blases = C.cast(blases, C.c_void_p)
+        tl, tp, inst = s.tlas()
+        oracle = lambda **k: O.trace_two_level(v, i, p, trees, inst, tl, tp, org, d, **k)  # noqa: E731
+    device.upload_geometry(g)
+    r, o = device.trace_closest(org, d, counters=True), oracle()
+    assert_same(r, o)
+    assert kind == "flat" or same_bits(r["instance"], o["instance"])
+    hidden = np.isfinite(r["t"]) & (r["triangle"] == -1)
+    assert 0.005 < hidden.mean() and (r["triangle"] >= 0).any()
+    a, o = device.trace_any(org, d, counters=True), oracle(occlusion=True)
+    assert np.array_equal(a["occluded"], o["occluded"]) and (a["occluded"][hidden] == 1).all()
+    assert_same(a, o, keys=("node_tests", "triangle_tests"))
+
+
 def test_launch_shape_invariance(device, tri_scene):
     org, d = workload_rays(tri_scene, n_random=30000, res=64)
     base = gpu_closest(device, tri_scene, org, d)

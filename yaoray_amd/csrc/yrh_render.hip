@@ -1699,6 +1699,10 @@ struct ShadowWalk {
         uint32_t occ = 1u;
         bool again = false;
         bool hit = best.Hit();
+        if (hit && best.id == -1) {  // a triangle without a flat index has no material: it blocks
+            P->s_occ[e] = 1u;
+            return false;
+        }
         if (kAlpha && hit && !trav::IsSphereId(best.id) &&
             !(HitAlpha(*S, *L, best.id, inst, best.u, best.v, XYZ(lo), XYZ(ld), best.t, nullptr) >= 0.5f)) {
             // TraceVisibleSurface's alpha skip within this segment
@@ -1859,7 +1863,7 @@ struct AlphaPath {
     __device__ __forceinline__ bool Finish(int32_t ray, const trav::Best& best, int32_t inst, uint32_t, uint32_t,
                                            uint32_t, const float4& lo, const float4& ld, float4& next_org,
                                            float4& next_dir) const {
-        bool hit = best.Hit();
+        bool hit = best.Hit() && best.id != -1;  // shading takes -1 as a miss
         if (hit && !trav::IsSphereId(best.id)) {
             const float4* df = diff != nullptr ? diff + 2 * q_path[ray] : nullptr;
             if (!(HitAlpha(*S, *L, best.id, inst, best.u, best.v, XYZ(lo), XYZ(ld), best.t, df) >= 0.5f)) {
@@ -1875,7 +1879,8 @@ struct AlphaPath {
                 hit = false;
             }
         }
-        a->hit[ray] = make_float4(best.t, best.u, best.v, __int_as_float(hit ? best.id : -1));
+        const float4 record = best.Record();
+        a->hit[ray] = make_float4(record.x, record.y, record.z, __int_as_float(hit ? best.id : -1));
         if (a->inst_out != nullptr) a->inst_out[ray] = hit ? inst : -1;
         return false;
     }

@@ -160,13 +160,21 @@ __device__ __forceinline__ bool Slab(const RayPre& r, float lx, float ly, float 
     return t_max >= t_min;
 }
 
-// The closest hit so far: id -1 = none.
+// The closest hit so far. u holds kNoHitU until there is one: every id is a
+// valid hit (flat triangle indices come from the caller, -1 among them), and an
+// accepted triangle's u is at least 0 or NaN, a sphere's never near -1.
+constexpr float kNoHitU = -1.0f;
 struct Best {
     float t;
     float u;
     float v;
     int32_t id;
-    __device__ __forceinline__ bool Hit() const { return id != -1; }
+    static __device__ __forceinline__ Best None(float t) { return Best{t, kNoHitU, 0.0f, -1}; }
+    __device__ __forceinline__ bool Hit() const { return u != kNoHitU; }
+    // The hit record: (t, u, v, id), u = v = 0 and id = -1 without a hit.
+    __device__ __forceinline__ float4 Record() const {
+        return make_float4(t, Hit() ? u : 0.0f, v, __int_as_float(id));
+    }
 };
 
 // IntersectTriangle on a (p0, e1, e2) slot. Returns true when `best` changed.
@@ -418,7 +426,7 @@ struct RayArrayPolicy {
         if (kAny) {
             a->occluded[ray] = best.Hit() ? 1u : 0u;
         } else {
-            a->hit[ray] = make_float4(best.t, best.u, best.v, __int_as_float(best.id));
+            a->hit[ray] = best.Record();
             if (a->inst_out != nullptr) a->inst_out[ray] = best.Hit() ? inst : -1;
         }
         if (a->node_tests != nullptr) a->node_tests[ray] = nt;
@@ -555,14 +563,14 @@ __device__ __forceinline__ void TraceFlatLoop(const TraceArgs& a, const Policy& 
     int32_t ray = -1;
     float dx = 0, dy = 0, dz = 0, t_min = 0;
     RayPre pre{};
-    Best best{0, 0, 0, -1};
+    Best best = Best::None(0.0f);
     uint32_t nt = 0, tt = 0, ts = 0;
     int32_t cur = kNoRecord;  // this lane's next record
 
     auto start = [&](const float4& o4, const float4& d4) {
         t_min = o4.w;
         dx = d4.x; dy = d4.y; dz = d4.z;
-        best = Best{d4.w, 0.0f, 0.0f, -1};
+        best = Best::None(d4.w);
         nt = 0;
         tt = 0;
         ts = 0;
@@ -657,21 +665,21 @@ __device__ __forceinline__ void TraceTwoLevelLoop(const TraceArgs& a, const Poli
     // its direction.
     RayPre pre{};
     float tdx = 0, tdy = 0, tdz = 0;
-    Best best{0, 0, 0, -1};
+    Best best = Best::None(0.0f);
     int32_t best_inst = -1;
     uint32_t nt = 0, tt = 0, ts = 0;
     // The BLAS being traversed: its hit, and the stack level below it.
     bool in_blas = false;
     uint32_t blas_base = 0;
     int32_t cur_inst = -1;
-    Best bbest{0, 0, 0, -1};
+    Best bbest = Best::None(0.0f);
     int32_t cur = kNoRecord;   // this lane's next record
     int32_t inst = kNoRecord;  // the next instance slot of the TLAS leaf being expanded
 
     auto start = [&](const float4& o4, const float4& d4) {
         ox = o4.x; oy = o4.y; oz = o4.z; t_min = o4.w;
         dx = d4.x; dy = d4.y; dz = d4.z;
-        best = Best{d4.w, 0.0f, 0.0f, -1};
+        best = Best::None(d4.w);
         best_inst = -1;
         nt = 0;
         tt = 0;
@@ -778,7 +786,7 @@ __device__ __forceinline__ void TraceTwoLevelLoop(const TraceArgs& a, const Poli
                             // The root's entry distance is within [t_min, best t], so the
                             // stack pop it replaces would always have taken it.
                             pre = bpre;
-                            bbest = Best{best.t, 0.0f, 0.0f, -1};
+                            bbest = Best::None(best.t);
                             blas_base = st.sp;
                             in_blas = true;
                             cur = root & ~kInstanceBit;
