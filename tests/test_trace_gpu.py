@@ -183,6 +183,62 @@ def test_leaves_that_share_primitives(device, kind):
     assert (r["triangle"] >= 0).any()
 
 
+def test_leaves_that_name_the_same_range_share_slots(device):
+    """512 leaves over the same 1000 primitives: their slots are held once (25 MB
+    otherwise), and every leaf finds them."""
+    import torch
+
+    from yaoray_amd.api import BvhArrays
+    s = Scene.triangles(1000, seed=3)
+    s.build_accel()
+    v, i, p = s.geometry()
+    b = s.flat_bvh()
+    nodes = []
+
+    def add(levels):
+        nodes.append(b.nodes[0].copy())
+        k = len(nodes) - 1
+        if levels == 0:
+            nodes[k]["payload_offset"], nodes[k]["primitive_count"] = 0, len(b.primitive_indices)
+            return
+        add(levels - 1)
+        nodes[k]["payload_offset"], nodes[k]["primitive_count"] = len(nodes), 0
+        add(levels - 1)
+
+    add(9)
+    t = BvhArrays(np.array(nodes), b.primitive_indices, b.primitives, 10)
+    g = s.geometry_desc()
+    device.upload_geometry(g)
+    device.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    g.flat = t.desc()
+    device.upload_geometry(g)
+    assert before - torch.cuda.mem_get_info()[0] < 8 << 20
+    org, d = random_rays(64, seed=12)
+    assert_same(device.trace_closest(org, d, counters=True), O.trace_flat(v, i, p, t, org, d))
+
+
+def test_upload_time_is_linear_in_the_number_of_meshes(device):
+    """6000 meshes of 100 triangles, 0.06 s (2.7 s where each mesh moves all those
+    before it; 12000 meshes took 40 s)."""
+    import time
+
+    from yaoray_amd.api import PRIMITIVE_DTYPE, VERTEX_DTYPE
+    meshes, tris = 6000, 100
+    rng = np.random.default_rng(2)
+    v = np.zeros(meshes * tris * 3, VERTEX_DTYPE)
+    v["position"] = (rng.uniform(-1, 1, (meshes * tris, 1, 3)) + rng.uniform(-0.1, 0.1, (meshes * tris, 3, 3))).reshape(-1, 3)
+    p = np.zeros(meshes, PRIMITIVE_DTYPE)
+    p["first_index"], p["index_count"] = np.arange(meshes) * 3 * tris, 3 * tris
+    s = Scene.from_arrays(v, np.arange(len(v), dtype=np.uint32), p, np.arange(meshes, dtype=np.int32),
+                          np.stack([trs((0, 0, 0), (0, 1, 0), 0, 1.0)] * meshes))
+    s.build_accel()
+    assert s.info.blas_count == 6000
+    t = time.perf_counter()
+    device.upload_scene(s)
+    assert time.perf_counter() - t < 1.0
+
+
 @pytest.mark.parametrize("kind", ["flat", "two_level"])
 def test_hits_on_triangles_without_a_flat_index(device, kind):
     """A caller's tree may hold triangles whose flat index is -1: they shorten

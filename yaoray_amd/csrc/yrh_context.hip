@@ -6,7 +6,9 @@
 #include <cmath>
 #include <cstring>
 #include <limits>
+#include <map>
 #include <new>
+#include <utility>
 
 namespace yrh {
 
@@ -40,8 +42,7 @@ namespace {
 // ResolveCode turns the indices into arena units.
 struct PackedBvh {
     std::vector<DevNode> nodes;
-    std::vector<float4> slots;        // three per slot
-    std::vector<int32_t> slot_source;  // per slot: its position in primitive_indices
+    std::vector<float4> slots;  // three per slot
     int32_t root_code = 0;
     float root_lo[3] = {0, 0, 0};
     float root_hi[3] = {0, 0, 0};
@@ -154,59 +155,90 @@ int ValidateGeometry(const yrh_geometry_desc* g, std::string& error) {
 }
 
 // Validates one reference BVH and appends its repacked form to `out`: interior
-// nodes in the reference's order, and each leaf's slots one after another
-// (leaves may share primitives). `slot_payload(prim, dst)` writes the three
-// float4 of a slot; the second one's .w is the leaf-end mark, set here.
+// nodes in the reference's order, and a slot per primitive_indices position,
+// which leaves name in place, so ones that share primitives share slots. Only
+// a leaf with another's end inside its range (its marks would end it there)
+// gets slots of its own, past the positions. `slot_payload(position, prim, dst)`
+// writes the three float4 of a slot; the second one's .w is the leaf-end mark,
+// set here.
 template <typename SlotFn>
 bool PackBvh(const yrh_bvh_desc& bvh, PackedBvh& out, std::string& error, SlotFn&& slot_payload) {
     if (!ValidateBvh(bvh, error)) return false;
-    const int64_t slot_base = static_cast<int64_t>(out.slot_source.size());
-    if (slot_base + bvh.primitive_index_count > kMaxSlot) {
+    const size_t slot_base = out.slots.size() / 3;
+    const size_t positions = static_cast<size_t>(bvh.primitive_index_count);
+    if (slot_base + positions > static_cast<size_t>(kMaxSlot)) {
         error = "too many BVH primitive slots for the device layout";
         return false;
     }
-    std::vector<float4> payload(3 * static_cast<size_t>(bvh.primitive_index_count));
-    for (int32_t s = 0; s < bvh.primitive_index_count; ++s) {
+    out.slots.resize(3 * (slot_base + positions));
+    for (size_t s = 0; s < positions; ++s) {
         const int32_t p = bvh.primitive_indices[s];
         if (p < 0 || p >= bvh.primitive_count) {
             error = "BVH primitive index out of bounds";
             return false;
         }
-        if (!slot_payload(bvh.primitives[p], &payload[3 * static_cast<size_t>(s)], error)) return false;
+        float4* dst = &out.slots[3 * (slot_base + s)];
+        if (!slot_payload(static_cast<int32_t>(s), bvh.primitives[p], dst, error)) return false;
+        dst[1].w = IntBits(0);
     }
+    // Leaf-end marks, and their number before each position.
     std::vector<int32_t> code(static_cast<size_t>(bvh.node_count));
+    std::vector<uint8_t> ends(positions, 0);
     int64_t interior = static_cast<int64_t>(out.nodes.size());
-    int64_t slots = slot_base;
     for (int32_t i = 0; i < bvh.node_count; ++i) {
         const yrh_bvh_node& n = bvh.nodes[i];
         if (n.primitive_count > 0) {
-            code[static_cast<size_t>(i)] = kLeafBit | static_cast<int32_t>(slots);
-            slots += n.primitive_count;
+            ends[static_cast<size_t>(n.payload_offset) + static_cast<size_t>(n.primitive_count) - 1] = 1;
         } else {
             code[static_cast<size_t>(i)] = static_cast<int32_t>(interior++);
         }
-        if (kNodeUnits * interior + kSlotUnits * slots > kMaxUnits) {
-            error = "too many BVH primitive slots for the device layout";
-            return false;
-        }
     }
-    out.nodes.resize(static_cast<size_t>(interior));
-    out.slots.reserve(3 * static_cast<size_t>(slots));
-    out.slot_source.reserve(static_cast<size_t>(slots));
+    if (kNodeUnits * interior > kMaxUnits) {
+        error = "too many BVH nodes for the device layout";
+        return false;
+    }
+    std::vector<int32_t> ends_before(positions);
+    int32_t count = 0;
+    for (size_t s = 0; s < positions; ++s) {
+        ends_before[s] = count;
+        count += ends[s];
+        if (ends[s] != 0) out.slots[3 * (slot_base + s) + 1].w = IntBits(1);
+    }
+    std::map<std::pair<int32_t, int32_t>, int32_t> own;  // ranges with slots of their own: their code
     for (int32_t i = 0; i < bvh.node_count; ++i) {
         const yrh_bvh_node& n = bvh.nodes[i];
-        if (n.primitive_count > 0) {
-            for (int32_t k = 0; k < n.primitive_count; ++k) {
-                const int32_t s = n.payload_offset + k;
-                const float4* src = &payload[3 * static_cast<size_t>(s)];
-                const float last = IntBits(k + 1 == n.primitive_count ? 1 : 0);
-                out.slots.push_back(src[0]);
-                out.slots.push_back(make_float4(src[1].x, src[1].y, src[1].z, last));
-                out.slots.push_back(src[2]);
-                out.slot_source.push_back(s);
+        if (n.primitive_count <= 0) continue;
+        const size_t first = static_cast<size_t>(n.payload_offset);
+        const size_t last = first + static_cast<size_t>(n.primitive_count) - 1;
+        int32_t slot = static_cast<int32_t>(slot_base + first);
+        if (ends_before[first] != ends_before[last]) {
+            const auto known = own.find({n.payload_offset, n.primitive_count});
+            if (known != own.end()) {
+                slot = known->second;
+            } else {
+                const size_t begin = out.slots.size() / 3;
+                if (begin + static_cast<size_t>(n.primitive_count) > static_cast<size_t>(kMaxSlot)) {
+                    error = "too many BVH primitive slots for the device layout";
+                    return false;
+                }
+                out.slots.resize(out.slots.size() + 3 * static_cast<size_t>(n.primitive_count));
+                for (size_t s = first; s <= last; ++s) {
+                    const float4* src = &out.slots[3 * (slot_base + s)];
+                    float4* dst = &out.slots[3 * (begin + s - first)];
+                    dst[0] = src[0];
+                    dst[1] = make_float4(src[1].x, src[1].y, src[1].z, IntBits(s == last ? 1 : 0));
+                    dst[2] = src[2];
+                }
+                slot = static_cast<int32_t>(begin);
+                own.emplace(std::make_pair(n.payload_offset, n.primitive_count), slot);
             }
-            continue;
         }
+        code[static_cast<size_t>(i)] = kLeafBit | slot;
+    }
+    out.nodes.resize(static_cast<size_t>(interior));
+    for (int32_t i = 0; i < bvh.node_count; ++i) {
+        const yrh_bvh_node& n = bvh.nodes[i];
+        if (n.primitive_count > 0) continue;
         const yrh_bvh_node& l = bvh.nodes[i + 1];
         const yrh_bvh_node& r = bvh.nodes[n.payload_offset];
         DevNode& rec = out.nodes[static_cast<size_t>(code[static_cast<size_t>(i)])];
@@ -232,7 +264,7 @@ bool PackBvh(const yrh_bvh_desc& bvh, PackedBvh& out, std::string& error, SlotFn
 // test rejects, so it is counted but never hit, as in the reference.
 struct TriangleSlotWriter {
     const yrh_geometry_desc* g;
-    bool operator()(const yrh_bvh_primitive& prim, float4* dst, std::string& error) const {
+    bool operator()(int32_t, const yrh_bvh_primitive& prim, float4* dst, std::string& error) const {
         if (prim.kind == 1) {
             // Sphere slot: (centre, -2 - sphere) (radius, 0, 0, 0) (0, 0, 0, 0).
             // A bad handle (skipped by the reference, bvh_traversal.cpp:130-133)
@@ -554,21 +586,21 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
             if (bi < 0 || bi >= g->blas_count) return Fail(ctx, YRH_E_INVALID_ARGUMENT, "instance BLAS out of bounds");
             resolved[static_cast<size_t>(s)] = tp.instance;
         }
-        // PackBvh gives the nodes and, per slot, its position; the instance
-        // slots are filled from those.
+        // PackBvh gives the nodes and slots that hold their position; the
+        // instance slots are filled from those.
         std::vector<yrh_bvh_primitive> dummy(static_cast<size_t>(std::max(1, g->tlas_primitive_count)));
         yrh_bvh_desc tdesc = t;
         tdesc.primitives = dummy.data();
         tdesc.primitive_count = static_cast<int32_t>(dummy.size());
-        const auto no_slot = [](const yrh_bvh_primitive&, float4* dst, std::string&) {
-            dst[0] = dst[1] = dst[2] = make_float4(0, 0, 0, 0);
+        const auto position_slot = [](int32_t position, const yrh_bvh_primitive&, float4* dst, std::string&) {
+            dst[0] = dst[1] = dst[2] = make_float4(IntBits(position), 0.0f, 0.0f, 0.0f);
             return true;
         };
-        if (!PackBvh(tdesc, tl, error, no_slot)) return Fail(ctx, YRH_E_INVALID_ARGUMENT, error);
+        if (!PackBvh(tdesc, tl, error, position_slot)) return Fail(ctx, YRH_E_INVALID_ARGUMENT, error);
         const int64_t slot_base = static_cast<int64_t>(packed.nodes.size() + tl.nodes.size()) * kNodeUnits;
-        instances.resize(tl.slot_source.size());
+        instances.resize(tl.slots.size() / 3);
         for (size_t s = 0; s < instances.size(); ++s) {
-            const int32_t i = resolved[static_cast<size_t>(tl.slot_source[s])];
+            const int32_t i = resolved[static_cast<size_t>(FloatBits(tl.slots[3 * s].x))];
             const int32_t last = FloatBits(tl.slots[3 * s + 1].w) != 0 ? kInstanceBit : 0;
             DevInstanceSlot& d = instances[s];
             if (i <= -2) {
