@@ -49,9 +49,9 @@ struct PackedBvh {
     bool empty = true;
 };
 
-int32_t ResolveCode(int32_t code, int64_t node_base, int64_t leaf_base, int32_t slot_units, int32_t leaf_bits) {
-    if (code >= 0) return static_cast<int32_t>((node_base + code) * kNodeUnits);
-    return leaf_bits | static_cast<int32_t>(leaf_base + static_cast<int64_t>(code & ~kLeafBit) * slot_units);
+int32_t ResolveCode(int32_t code, int64_t node_base, int64_t slot_base, int32_t slot_units) {
+    if (code >= 0) return static_cast<int32_t>(node_base + static_cast<int64_t>(code) * kNodeUnits);
+    return kLeafBit | static_cast<int32_t>(slot_base + static_cast<int64_t>(code & ~kLeafBit) * slot_units);
 }
 
 float IntBits(int32_t v) {
@@ -597,11 +597,11 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
             return true;
         };
         if (!PackBvh(tdesc, tl, error, position_slot)) return Fail(ctx, YRH_E_INVALID_ARGUMENT, error);
-        const int64_t slot_base = static_cast<int64_t>(packed.nodes.size() + tl.nodes.size()) * kNodeUnits;
+        const int64_t slot_base = static_cast<int64_t>(packed.nodes.size()) * kNodeUnits;
         instances.resize(tl.slots.size() / 3);
         for (size_t s = 0; s < instances.size(); ++s) {
             const int32_t i = resolved[static_cast<size_t>(FloatBits(tl.slots[3 * s].x))];
-            const int32_t last = FloatBits(tl.slots[3 * s + 1].w) != 0 ? kInstanceBit : 0;
+            const int32_t last = FloatBits(tl.slots[3 * s + 1].w) != 0 ? kLastInstanceBit : 0;
             DevInstanceSlot& d = instances[s];
             if (i <= -2) {
                 // TLAS sphere slot: r0 = (centre, radius), hi.w = -2 - sphere.
@@ -618,7 +618,7 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
             d.r1 = make_float4(m[1], m[5], m[9], m[13]);
             d.r2 = make_float4(m[2], m[6], m[10], m[14]);
             d.lo = root.lo;
-            d.lo.w = IntBits(ResolveCode(FloatBits(root.lo.w), 0, slot_base, kSlotUnits, kLeafBit) | last);
+            d.lo.w = IntBits(ResolveCode(FloatBits(root.lo.w), 0, slot_base, kSlotUnits) | last);
             d.hi = make_float4(root.hi.x, root.hi.y, root.hi.z, IntBits(i));
         }
         geo.stack_capacity = std::max(1, t.max_depth) + blas_depth + 3;
@@ -626,41 +626,38 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
         return Fail(ctx, YRH_E_INVALID_ARGUMENT, "unknown acceleration kind");
     }
 
-    // The arena: nodes (BLASes or the flat tree, then the TLAS), primitive
-    // slots, instance slots; indices become units.
+    // The arena; indices become units.
     {
-        const int64_t tlas_base = static_cast<int64_t>(packed.nodes.size());
-        const int64_t nodes = tlas_base + static_cast<int64_t>(tl.nodes.size());
-        const int64_t slot_base = nodes * kNodeUnits;
-        const int64_t inst_base = slot_base + static_cast<int64_t>(packed.slots.size());
-        const int64_t units = inst_base + static_cast<int64_t>(instances.size()) * kInstanceUnits;
-        if (units > kMaxUnits) return Fail(ctx, YRH_E_INVALID_ARGUMENT, "too many BVH primitive slots for the device layout");
-        const int32_t tlas_leaf = kLeafBit | kInstanceBit;
+        ArenaLayout at;
+        if (!LayOutArena(static_cast<int64_t>(packed.nodes.size()), static_cast<int64_t>(packed.slots.size()) / 3,
+                         static_cast<int64_t>(tl.nodes.size()), static_cast<int64_t>(instances.size()), at)) {
+            return Fail(ctx, YRH_E_INVALID_ARGUMENT, "too many BVH records for the device layout");
+        }
         for (DevNode& n : packed.nodes) {
-            n.d.x = ResolveCode(n.d.x, 0, slot_base, kSlotUnits, kLeafBit);
-            n.d.y = ResolveCode(n.d.y, 0, slot_base, kSlotUnits, kLeafBit);
+            n.d.x = ResolveCode(n.d.x, 0, at.slots, kSlotUnits);
+            n.d.y = ResolveCode(n.d.y, 0, at.slots, kSlotUnits);
         }
         for (DevNode& n : tl.nodes) {
-            n.d.x = ResolveCode(n.d.x, tlas_base, inst_base, kInstanceUnits, tlas_leaf);
-            n.d.y = ResolveCode(n.d.y, tlas_base, inst_base, kInstanceUnits, tlas_leaf);
+            n.d.x = ResolveCode(n.d.x, at.tlas_nodes, at.instances, kInstanceUnits);
+            n.d.y = ResolveCode(n.d.y, at.tlas_nodes, at.instances, kInstanceUnits);
         }
         const bool two = g->accel_kind == YRH_ACCEL_TWO_LEVEL;
         const PackedBvh& top = two ? tl : packed;
         geo.empty = top.empty;
-        geo.root_code = two ? ResolveCode(tl.root_code, tlas_base, inst_base, kInstanceUnits, tlas_leaf)
-                            : ResolveCode(packed.root_code, 0, slot_base, kSlotUnits, kLeafBit);
+        geo.root_code = two ? ResolveCode(tl.root_code, at.tlas_nodes, at.instances, kInstanceUnits)
+                            : ResolveCode(packed.root_code, 0, at.slots, kSlotUnits);
         std::memcpy(geo.root_lo, top.root_lo, sizeof(geo.root_lo));
         std::memcpy(geo.root_hi, top.root_hi, sizeof(geo.root_hi));
-        const size_t bytes = static_cast<size_t>(std::max<int64_t>(units, 1)) * sizeof(float4);
+        const size_t bytes = static_cast<size_t>(std::max<int64_t>(at.units, 1)) * sizeof(float4);
         if ((rc = CheckHip(ctx, hipMalloc(&geo.arena.ptr, bytes), "hipMalloc")) != YRH_OK) return rc;
         geo.arena.bytes = bytes;
         float4* base = geo.arena.as<float4>();
         if ((rc = yrh_copy_to_device(ctx, base, packed.nodes.data(), packed.nodes.size() * sizeof(DevNode))) != YRH_OK ||
-            (rc = yrh_copy_to_device(ctx, base + tlas_base * kNodeUnits, tl.nodes.data(),
+            (rc = yrh_copy_to_device(ctx, base + at.tlas_nodes, tl.nodes.data(),
                                      tl.nodes.size() * sizeof(DevNode))) != YRH_OK ||
-            (rc = yrh_copy_to_device(ctx, base + slot_base, packed.slots.data(),
+            (rc = yrh_copy_to_device(ctx, base + at.slots, packed.slots.data(),
                                      packed.slots.size() * sizeof(float4))) != YRH_OK ||
-            (rc = yrh_copy_to_device(ctx, base + inst_base, instances.data(),
+            (rc = yrh_copy_to_device(ctx, base + at.instances, instances.data(),
                                      instances.size() * sizeof(DevInstanceSlot))) != YRH_OK) {
             return rc;
         }

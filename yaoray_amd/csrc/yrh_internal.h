@@ -9,8 +9,8 @@
 //     node_tests counter are unchanged. Only interior nodes have a record
 //     (half of a binary tree's nodes are leaves), in the reference's order.
 //   * A child is named by a 32-bit code: >= 0 is an interior node's unit;
-//     < 0 a leaf: bit 31 set, bits 0..29 the unit of its first slot, bit 30
-//     set for a TLAS leaf (instance slots). kNoRecord names nothing.
+//     < 0 a leaf: bit 31 set, the others the unit of its first slot.
+//     kNoRecord names nothing.
 //   * Primitive slots follow the nodes, each leaf's in leaf order; a slot
 //     holds the triangle as (p0, flat triangle index) (e1 = p1 - p0, last)
 //     (e2 = p2 - p0, 0): 48 bytes, one coalesced fetch per test in place of
@@ -18,7 +18,8 @@
 //     1 in the leaf's last slot, so a leaf needs no count. e1/e2 are the same
 //     IEEE subtractions the reference performs per test, so every
 //     intersection is bit-identical.
-//   * Instance slots (two-level scenes) come last, 80 bytes each.
+//   * In two-level scenes that part holds every BLAS; the TLAS nodes and the
+//     instance slots, 80 bytes each, follow it.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -53,10 +54,27 @@ constexpr int32_t kNodeUnits = 4;
 constexpr int32_t kSlotUnits = 3;
 constexpr int32_t kInstanceUnits = 5;
 constexpr int32_t kLeafBit = static_cast<int32_t>(0x80000000u);
-constexpr int32_t kInstanceBit = 0x40000000;
-constexpr int32_t kUnitMask = 0x3fffffff;
+constexpr int32_t kLastInstanceBit = 0x40000000;  // of an instance slot's BLAS root code
+constexpr int32_t kUnitMask = 0x7fffffff;
 constexpr int32_t kNoRecord = 0x7fffffff;
-constexpr int64_t kMaxUnits = int64_t{1} << 30;
+constexpr int64_t kMaxUnits = int64_t{1} << 31;
+constexpr int64_t kMaxBlasUnits = int64_t{1} << 30;  // a BLAS root code leaves bit 30 free
+
+// Where the arena's parts begin (units): BLAS (or flat) nodes at 0, their
+// slots, the TLAS nodes, the instance slots.
+struct ArenaLayout {
+    int64_t slots = 0, tlas_nodes = 0, instances = 0, units = 0;
+};
+// False: a code could not name every record. Trees whose leaves share no
+// primitives fit up to kMaxSlot slots in all BLASes and as many in the TLAS.
+inline bool LayOutArena(int64_t nodes, int64_t slots, int64_t tlas_nodes, int64_t instance_slots, ArenaLayout& a) {
+    a.slots = nodes * kNodeUnits;
+    const int64_t end = a.slots + slots * kSlotUnits;
+    a.tlas_nodes = (end + kNodeUnits - 1) / kNodeUnits * kNodeUnits;  // whole 64-byte lines
+    a.instances = a.tlas_nodes + tlas_nodes * kNodeUnits;
+    a.units = a.instances + instance_slots * kInstanceUnits;
+    return a.units <= kMaxUnits && (tlas_nodes + instance_slots == 0 || end <= kMaxBlasUnits);
+}
 
 struct alignas(16) DevNode {
     float4 a;  // L.min.x L.min.y L.min.z L.max.x
@@ -74,12 +92,12 @@ struct alignas(16) DevBlasRoot {
 
 // One TLAS leaf slot: the instance's world-to-object rows and its BLAS root,
 // so a traversal step into an instance is one 80-byte fetch. The root code's
-// bit 30 is set in the last slot of a leaf.
+// kLastInstanceBit is set in the last slot of a leaf.
 struct alignas(16) DevInstanceSlot {
     float4 r0;  // world_to_object m[0], m[4], m[8],  m[12]
     float4 r1;  //                 m[1], m[5], m[9],  m[13]
     float4 r2;  //                 m[2], m[6], m[10], m[14]
-    float4 lo;  // BLAS root box min, w = root code bits (bit 30: last slot of the leaf)
+    float4 lo;  // BLAS root box min, w = root code bits, kLastInstanceBit
     float4 hi;  // BLAS root box max, w = instance index bits
 };
 static_assert(sizeof(DevInstanceSlot) == 80, "instance slot record is 80 bytes");

@@ -761,7 +761,7 @@ __device__ __forceinline__ void TraceTwoLevelLoop(const TraceArgs& a, const Poli
                     const DevInstanceSlot m = *reinterpret_cast<const DevInstanceSlot*>(Record(a.arena, inst));
                     const int32_t slot_id = __float_as_int(m.hi.w);
                     const int32_t root = __float_as_int(m.lo.w);
-                    inst = NextSlot(inst, kInstanceUnits, (root & kInstanceBit) != 0);
+                    inst = NextSlot(inst, kInstanceUnits, (root & kLastInstanceBit) != 0);
                     if (kSpheres && IsSphereId(slot_id)) {
                         // A TLAS sphere (IntersectTlasSphere, two_level_bvh.cpp:231-253):
                         // tested against the world ray, no instance.
@@ -789,7 +789,7 @@ __device__ __forceinline__ void TraceTwoLevelLoop(const TraceArgs& a, const Poli
                             bbest = Best::None(best.t);
                             blas_base = st.sp;
                             in_blas = true;
-                            cur = root & ~kInstanceBit;
+                            cur = root & ~kLastInstanceBit;
                         }
                     }
                 }
