@@ -1,4 +1,4 @@
-"""Large host copies go through pinned buffers on several threads: every byte
+"""Large copies to the host go through pinned buffers on several threads: every byte
 arrives, in both directions, at sizes around the chunk and thread limits."""
 import numpy as np
 import pytest
@@ -31,3 +31,31 @@ def test_large_copies_arrive_whole(nbytes):
         buf.free()
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("mib", [8, 16])
+def test_uploads_cost_no_more_than_a_plain_copy(mib):
+    """Scene arrays of some MiB to the device, against torch's copy of the same
+    pageable memory (through the context's pinned buffers they took 1.3 to 1.4
+    times as long)."""
+    import time
+
+    import torch
+    a = np.ones(mib * MIB, np.uint8)
+    t, on_device = torch.from_numpy(a), torch.empty(a.nbytes, dtype=torch.uint8, device="cuda")
+    dev = Device(0)
+    try:
+        buf = DeviceBuffer(dev, a.nbytes)
+        ours, plain = [], []
+        for _ in range(30):
+            t0 = time.perf_counter()
+            buf.upload(a)
+            t1 = time.perf_counter()
+            on_device.copy_(t)
+            torch.cuda.synchronize()
+            ours.append(t1 - t0)
+            plain.append(time.perf_counter() - t1)
+        buf.free()
+    finally:
+        dev.close()
+    assert np.median(ours) < 1.15 * np.median(plain)

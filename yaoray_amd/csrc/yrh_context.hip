@@ -420,10 +420,7 @@ int yrh_device_free(yrh_context* ctx, void* ptr) {
 int yrh_copy_to_device(yrh_context* ctx, void* dst, const void* src, size_t bytes) {
     if (ctx == nullptr || (bytes > 0 && (dst == nullptr || src == nullptr))) return YRH_E_INVALID_ARGUMENT;
     if (bytes == 0) return YRH_OK;
-    bool done = false;
-    int rc = StagedCopyToDevice(ctx, dst, src, bytes, &done);
-    if (done || rc != YRH_OK) return rc;
-    rc = CheckHip(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream), "hipMemcpyAsync H2D");
+    int rc = CheckHip(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream), "hipMemcpyAsync H2D");
     if (rc != YRH_OK) return rc;
     return CheckHip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
 }

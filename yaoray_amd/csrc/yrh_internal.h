@@ -199,7 +199,7 @@ struct yrh_context {
     void* noalloc_scratch = nullptr;
     yrh::RenderState* render = nullptr;  // surface/light data, film, path state (yrh_render.hip)
     yrh::GuideState* guide = nullptr;    // learned guiding proposal (yrh_guide.hip)
-    yrh::HostStage* stage = nullptr;     // pinned buffers of large host copies (yrh_stage.hip)
+    yrh::HostStage* stage = nullptr;     // pinned buffers of large copies to the host (yrh_stage.hip)
     bool large_copy_seen = false;
 };
 
@@ -258,11 +258,10 @@ int TracePhaseMs(yrh_context* ctx, float* order_ms, float* trace_ms);
 int UploadSurfaceGeometry(yrh_context* ctx, const yrh_geometry_desc* g);
 void DestroyRenderState(yrh_context* ctx);
 
-// Copies between pageable host memory and the device through the context's
-// pinned buffers (yrh_stage.hip), complete on return; *done false: not taken,
-// the caller copies plainly.
+// A copy from the device to pageable host memory through the context's pinned
+// buffers (yrh_stage.hip), complete on return; *done false: not taken, the
+// caller copies plainly.
 int StagedCopyToHost(yrh_context* ctx, void* dst, const void* src, size_t bytes, bool* done);
-int StagedCopyToDevice(yrh_context* ctx, void* dst, const void* src, size_t bytes, bool* done);
 void DestroyHostStage(yrh_context* ctx);
 
 // Guiding state for one render pass (yrh_guide.hip): fills `view` (mode off
