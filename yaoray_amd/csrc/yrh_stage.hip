@@ -49,11 +49,26 @@ void DestroyHostStage(yrh_context* ctx) {
 
 namespace {
 
-// The context's pinned buffers (16 MiB), or null: copies too small to gain,
+// The context's device as the current one while in scope: events belong to the
+// device that is current when they are made, and a copy leaves the caller's
+// choice as it was.
+struct DeviceScope {
+    int before = -1;
+    explicit DeviceScope(int device) {
+        if (hipGetDevice(&before) != hipSuccess) before = -1;
+        (void)hipSetDevice(device);
+    }
+    ~DeviceScope() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+    DeviceScope(const DeviceScope&) = delete;
+    DeviceScope& operator=(const DeviceScope&) = delete;
+};
+
+// The context's pinned buffers (16 MiB), or null:
 // a context's first copy unless it pays for the allocation by itself (a
 // context made for one frame reads one film), or no pinned memory to be had.
 HostStage* Stage(yrh_context* ctx, size_t bytes) {
-    if (bytes < kMinBytes) return nullptr;
     if (ctx->stage != nullptr) return ctx->stage;
     if (!ctx->large_copy_seen && bytes < (size_t{32} << 20)) {
         ctx->large_copy_seen = true;
@@ -91,14 +106,17 @@ void RunThreads(size_t chunks, const Work& work) {
 }  // namespace
 
 int StagedCopyToHost(yrh_context* ctx, void* dst, const void* src, size_t bytes, bool* done) {
+    *done = false;
+    if (bytes < kMinBytes) return YRH_OK;
+    const DeviceScope scope(ctx->device);
     HostStage* s = Stage(ctx, bytes);
-    *done = s != nullptr;
     if (s == nullptr) return YRH_OK;
+    *done = true;
     const size_t chunks = (bytes + kChunk - 1) / kChunk;
     std::atomic<size_t> next{0};
     std::atomic<int> status{hipSuccess};
     auto work = [&](int thread) {
-        (void)hipSetDevice(ctx->device);
+        if (thread != 0) (void)hipSetDevice(ctx->device);  // the caller's thread: done
         size_t held[2] = {chunks, chunks};  // the chunk in each of the thread's slots (chunks: none)
         for (int turn = 0;; turn ^= 1) {
             const int slot = 2 * thread + turn;
