@@ -65,6 +65,18 @@ struct DeviceScope {
     DeviceScope& operator=(const DeviceScope&) = delete;
 };
 
+// Whether the runtime knows nothing of p: pinned memory takes a plain copy at
+// the speed of the link (128 MiB in 2.4 ms, 4.4 ms through these buffers), and
+// device memory is not the host's to write.
+bool Pageable(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
 // The context's pinned buffers (16 MiB), or null:
 // a context's first copy unless it pays for the allocation by itself (a
 // context made for one frame reads one film), or no pinned memory to be had.
@@ -107,7 +119,7 @@ void RunThreads(size_t chunks, const Work& work) {
 
 int StagedCopyToHost(yrh_context* ctx, void* dst, const void* src, size_t bytes, bool* done) {
     *done = false;
-    if (bytes < kMinBytes) return YRH_OK;
+    if (bytes < kMinBytes || !Pageable(dst)) return YRH_OK;
     const DeviceScope scope(ctx->device);
     HostStage* s = Stage(ctx, bytes);
     if (s == nullptr) return YRH_OK;
