@@ -176,7 +176,7 @@ def program(tmp_path_factory):
     return str(d / "stage")
 
 
-@pytest.mark.parametrize("what", ["sizes", "device", "memory"])
+@pytest.mark.parametrize("what", ["sizes", "device", "memory", "failures"])
 def test_staged_copy(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
