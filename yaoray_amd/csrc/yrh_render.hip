@@ -203,7 +203,7 @@ struct RenderState {
     Slice s_org[2], s_dir[2], s_li[2], s_bsdf[2], s_nee[2], s_occ, s_trans;
     Slice l_state, l_med;
     bool cap_transparent = false;
-    bool two_shadow_queues = false;
+    std::vector<DevBuf> second;  // the odd bounces' shadow queue; empty: all bounces share the even one
     Slice counters;   // uint32[kCounterWords]
     DevBuf stats;     // uint64[kStatStride * kStatSlots]: kStatSlots copies of the statistics words
     // batched passes
@@ -2083,7 +2083,7 @@ int Grid(int64_t n, int block = kBlock) { return static_cast<int>(std::max<int64
 
 // The shadow queue of bounce `depth`.
 void SetShadowQueue(const RenderState& R, PassView& P, int depth) {
-    const int k = R.two_shadow_queues ? depth & 1 : 0;
+    const int k = R.second.empty() ? 0 : depth & 1;
     P.s_org = R.s_org[k].as<float4>();
     P.s_dir = R.s_dir[k].as<float4>();
     P.s_li = R.s_li[k].as<float4>();
@@ -2266,7 +2266,8 @@ __global__ void BsdfQueryKernel(const DevMaterial* mats, int64_t n, const int32_
 // Bytes per path slot and per shadow slot of the arrays EnsureCapacity
 // allocates, and per guided row (mixture + valid flag).
 constexpr size_t kPathSlotBytes = 4 + 4 + 4 + 16 + 16 + 16 + 16 + 4 + 16 + 16 + 16 + 2 * 16 + 2 * 16 + 2 * 4 + 16 + 4;
-constexpr size_t kShadowSlotBytes = 2 * 5 * 16 + 4;
+constexpr size_t kShadowQueueBytes = 5 * 16;  // and again for a second queue
+constexpr size_t kShadowSlotBytes = kShadowQueueBytes + 4;
 constexpr size_t kWalkSlotBytes = 16 + 4 + 16;  // transparent shadows only
 constexpr size_t kGuideRowBytes = yrg::kGuideMixtureRow * 4 + 4;
 
@@ -2284,10 +2285,34 @@ int EnsureDifferentials(yrh_context* ctx, RenderState& R) {
 // 1.5 GB or 256 MiB now and then takes the driver 39 ms to hand out.
 constexpr size_t kPassBlockBytes = size_t{64} << 20;
 
-// Allocates the pass buffers for `paths` path slots. Two shadow queues for
-// alternate bounces, or one (each Shade then waits for the Resolve before it)
-// without overlap, or where the second would take more than a quarter of the
-// memory left (the film, the guide's rows and the stack spill still need some).
+struct PassArray {
+    Slice* slice;
+    size_t bytes;
+};
+
+size_t PassPadded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
+// Allocates `arrays` one after another in blocks that are appended to `blocks`.
+int AllocPassArrays(yrh_context* ctx, const PassArray* arrays, size_t count, std::vector<DevBuf>& blocks) {
+    for (size_t k = 0; k < count;) {
+        size_t end = k, bytes = 0;
+        while (end < count && (end == k || bytes + PassPadded(arrays[end].bytes) <= kPassBlockBytes)) {
+            bytes += PassPadded(arrays[end].bytes);
+            ++end;
+        }
+        blocks.emplace_back();
+        const int rc = Alloc(ctx, blocks.back(), bytes);
+        if (rc != YRH_OK) return rc;
+        char* at = blocks.back().as<char>();
+        for (; k < end; ++k) {
+            arrays[k].slice->ptr = at;
+            at += PassPadded(arrays[k].bytes);
+        }
+    }
+    return YRH_OK;
+}
+
+// Allocates the pass buffers for `paths` path slots, with one shadow queue.
 int EnsureCapacity(yrh_context* ctx, RenderState& R, int64_t paths) {
     if (R.capacity >= paths && R.cap_shadow_slots >= R.shadow_slots && (R.cap_transparent || !R.transparent) &&
         R.counters.ptr != nullptr) {
@@ -2299,45 +2324,20 @@ int EnsureCapacity(yrh_context* ctx, RenderState& R, int64_t paths) {
     const size_t P = static_cast<size_t>(paths);
     const size_t S = static_cast<size_t>(R.shadow_slots) * P;
     const size_t W = R.transparent ? S : 1;  // transparent walks
-    struct Item {
-        Slice* slice;
-        size_t bytes;
-    } items[] = {
+    const PassArray arrays[] = {
         {&R.counters, 4 * kCounterWords},
-        {&R.p_pixel, 4 * P}, {&R.p_job, 4 * P}, {&R.p_sample, 4 * P}, {&R.p_tp, 16 * P}, {&R.p_rad, 16 * P}, {&R.p_prev, 16 * P}, {&R.p_flags, 4 * P},
-        {&R.p_med, 16 * P}, {&R.p_alb, 16 * P}, {&R.p_nrm, 16 * P}, {&R.p_dir, 16 * P},
+        {&R.p_pixel, 4 * P}, {&R.p_job, 4 * P}, {&R.p_sample, 4 * P}, {&R.p_tp, 16 * P}, {&R.p_rad, 16 * P},
+        {&R.p_prev, 16 * P}, {&R.p_flags, 4 * P}, {&R.p_med, 16 * P}, {&R.p_alb, 16 * P}, {&R.p_nrm, 16 * P},
+        {&R.p_dir, 16 * P},
         {&R.q_org[0], 16 * P}, {&R.q_org[1], 16 * P}, {&R.q_dir[0], 16 * P}, {&R.q_dir[1], 16 * P},
         {&R.q_path[0], 4 * P}, {&R.q_path[1], 4 * P}, {&R.hits, 16 * P}, {&R.hit_inst, 4 * P},
         {&R.s_occ, 4 * S}, {&R.s_trans, 16 * W}, {&R.l_state, 4 * W}, {&R.l_med, 16 * W},
         {&R.s_org[0], 16 * S}, {&R.s_dir[0], 16 * S}, {&R.s_li[0], 16 * S}, {&R.s_bsdf[0], 16 * S}, {&R.s_nee[0], 16 * S},
-        {&R.s_org[1], 16 * S}, {&R.s_dir[1], 16 * S}, {&R.s_li[1], 16 * S}, {&R.s_bsdf[1], 16 * S}, {&R.s_nee[1], 16 * S},
     };
-    constexpr size_t kSecondQueue = 5;  // the last items
-    auto padded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
-    const size_t first_count = std::size(items) - kSecondQueue;
-    size_t total = 0, second = 0;
-    for (size_t k = 0; k < std::size(items); ++k) (k < first_count ? total : second) += padded(items[k].bytes);
     R.capacity = 0;
+    R.second.clear();
     R.pass.clear();
-    size_t free_bytes = 0, device_bytes = 0;
-    if ((rc = CheckHip(ctx, hipMemGetInfo(&free_bytes, &device_bytes), "hipMemGetInfo")) != YRH_OK) return rc;
-    R.two_shadow_queues = ctx->render_overlap && free_bytes >= total && free_bytes - total >= 4 * second;
-    const size_t count = R.two_shadow_queues ? std::size(items) : first_count;
-    for (size_t k = count; k < std::size(items); ++k) items[k].slice->ptr = nullptr;
-    for (size_t k = 0; k < count;) {
-        size_t end = k, bytes = 0;
-        while (end < count && (end == k || bytes + padded(items[end].bytes) <= kPassBlockBytes)) {
-            bytes += padded(items[end].bytes);
-            ++end;
-        }
-        R.pass.emplace_back();
-        if ((rc = Alloc(ctx, R.pass.back(), bytes)) != YRH_OK) return rc;
-        char* at = R.pass.back().as<char>();
-        for (; k < end; ++k) {
-            items[k].slice->ptr = at;
-            at += padded(items[k].bytes);
-        }
-    }
+    if ((rc = AllocPassArrays(ctx, arrays, std::size(arrays), R.pass)) != YRH_OK) return rc;
     if (R.stats.ptr == nullptr) {
         if ((rc = Alloc(ctx, R.stats, kStatBytes)) != YRH_OK) return rc;
         if ((rc = CheckHip(ctx, hipMemsetAsync(R.stats.ptr, 0, kStatBytes, ctx->stream), "hipMemsetAsync")) != YRH_OK) {
@@ -2349,6 +2349,28 @@ int EnsureCapacity(yrh_context* ctx, RenderState& R, int64_t paths) {
     R.cap_shadow_slots = R.shadow_slots;
     R.cap_transparent = R.transparent;
     return rc != YRH_OK ? rc : EnsureDifferentials(ctx, R);
+}
+
+// A shadow queue of their own for odd bounces, so that Shade need not wait for
+// the Resolve just before it (LaunchPassSequence). Asked for by each overlapped
+// pass once everything else that it needs is there; given if it takes no more
+// than a quarter of the memory left.
+int EnsureSecondQueue(yrh_context* ctx, RenderState& R) {
+    if (!ctx->render_overlap || !R.second.empty()) return YRH_OK;
+    const size_t S = static_cast<size_t>(R.cap_shadow_slots) * static_cast<size_t>(R.capacity);
+    const PassArray arrays[] = {
+        {&R.s_org[1], 16 * S}, {&R.s_dir[1], 16 * S}, {&R.s_li[1], 16 * S}, {&R.s_bsdf[1], 16 * S}, {&R.s_nee[1], 16 * S},
+    };
+    size_t bytes = 0;
+    for (const PassArray& a : arrays) bytes += PassPadded(a.bytes);
+    size_t free_bytes = 0, device_bytes = 0;
+    const int rc = CheckHip(ctx, hipMemGetInfo(&free_bytes, &device_bytes), "hipMemGetInfo");
+    if (rc != YRH_OK || free_bytes / 4 < bytes) return rc;
+    if (AllocPassArrays(ctx, arrays, std::size(arrays), R.second) != YRH_OK) {
+        (void)hipGetLastError();
+        R.second.clear();
+    }
+    return YRH_OK;
 }
 
 // The second stream and the events of overlapped bounces.
@@ -2368,6 +2390,22 @@ int EnsureOverlap(yrh_context* ctx) {
     return YRH_OK;
 }
 
+// Sizes the traversal scratch of a pass over `paths` path slots for the streams
+// it uses: nothing may allocate once its kernels are being launched (or captured).
+int EnsureTraceScratch(yrh_context* ctx, RenderState& R, int64_t paths, bool overlap) {
+    TraceRequest r;
+    r.org = R.q_org[0].as<float4>();
+    r.dir = R.q_dir[0].as<float4>();
+    r.n_device = BounceSlot(R.counters.as<uint32_t>(), 0) + kCountQueue;
+    r.capacity = paths;
+    trav::TraceArgs a;
+    int grid = 0, block = 0, rc;
+    if ((rc = PrepareTraceArgs(ctx, r, a, grid, block)) != YRH_OK || !overlap) return rc;
+    if ((rc = EnsureOverlap(ctx)) != YRH_OK) return rc;
+    r.aux = true;
+    return PrepareTraceArgs(ctx, r, a, grid, block);
+}
+
 // Raygen and the bounces of one pass over `paths` path slots (the queue
 // capacity; the kernels read the live counts from the counter words).
 int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, const SurfaceView& S, const LightView& L,
@@ -2383,14 +2421,10 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
     // same. A walk through glass ends with a few long rays, which stood in the
     // way of every bounce: 8 instanced cameras 43.3 -> 34.4 ms (one stream
     // before), Cornell frame 1.96 -> 1.88 ms, textured frame 5.65 -> 5.56 ms.
-    hipStream_t ss = st;
-    if (overlap) {
-        if ((rc = EnsureOverlap(ctx)) != YRH_OK) return rc;
-        ss = ctx->aux_stream;
-    }
+    hipStream_t ss = overlap ? ctx->aux_stream : st;
     hipEvent_t shaded = ctx->bounce_events[0];
     hipEvent_t* resolved = ctx->bounce_events + 1;
-    const int lag = GV.rec != nullptr || !R.two_shadow_queues ? 1 : 2;
+    const int lag = GV.rec != nullptr || R.second.empty() ? 1 : 2;
     {
         const StageRange r("raygen");
         hipLaunchKernelGGL(RaygenKernel, dim3(Grid(paths)), dim3(kBlock), 0, st, P);
@@ -3080,8 +3114,8 @@ int yrh_suggest_paths_per_pass(yrh_context* ctx, int32_t max_depth, int64_t* pat
     // Per path: the path slot state (EnsureCapacity) and its shadow slots.
     const int shadow_slots = ctx->render != nullptr ? ctx->render->shadow_slots : 2;
     const bool transparent = ctx->render == nullptr || ctx->render->transparent;
-    size_t per_path = kPathSlotBytes +
-                      static_cast<size_t>(shadow_slots) * (kShadowSlotBytes + (transparent ? kWalkSlotBytes : 0));
+    size_t per_path = kPathSlotBytes + static_cast<size_t>(shadow_slots) *
+                                           (kShadowSlotBytes + kShadowQueueBytes + (transparent ? kWalkSlotBytes : 0));
     if (ctx->guide != nullptr) per_path += kGuideRowBytes + 64 * static_cast<size_t>(std::max(1, max_depth));
     const size_t held = ctx->render != nullptr ? static_cast<size_t>(ctx->render->capacity) * per_path : 0;
     const int64_t fit = static_cast<int64_t>((free_bytes + held) / 2 / per_path);
@@ -3110,13 +3144,15 @@ int yrh_render_pass(yrh_context* ctx, const yrh_render_desc* d) {
     (void)hipSetDevice(ctx->device);
     int rc = EnsureCapacity(ctx, R, paths);
     if (rc != YRH_OK) return rc;
+    const int max_depth = std::max(1, d->max_depth);
+    yrg::GuideView GV;
+    if ((rc = GuidePrepareView(ctx, paths, max_depth, &GV)) != YRH_OK) return rc;
+    if ((rc = EnsureTraceScratch(ctx, R, paths, ctx->render_overlap)) != YRH_OK) return rc;
+    if ((rc = EnsureSecondQueue(ctx, R)) != YRH_OK) return rc;
     PassView P = MakePassView(R, *d);
     const SurfaceView S = MakeSurfaceView(R);
     const LightView L = MakeLightView(R);
     hipStream_t st = ctx->stream;
-    const int max_depth = std::max(1, d->max_depth);
-    yrg::GuideView GV;
-    if ((rc = GuidePrepareView(ctx, paths, max_depth, &GV)) != YRH_OK) return rc;
     if ((rc = LaunchPassSequence(ctx, R, P, S, L, GV, paths, max_depth, ctx->render_overlap)) != YRH_OK) return rc;
     hipLaunchKernelGGL(AccumulateKernel, dim3(Grid(npix)), dim3(kBlock), 0, st, P);
     return CheckHip(ctx, hipGetLastError(), "render pass launch");
@@ -3228,6 +3264,11 @@ int yrh_batch_render(yrh_context* ctx, const yrh_batch_desc* d, float* job_ms, i
     rd.width = 1;
     rd.height = 1;
     rd.spp = 1;
+    const int max_depth = std::max(1, d->max_depth);
+    yrg::GuideView GV;
+    if ((rc = GuidePrepareView(ctx, capacity, max_depth, &GV)) != YRH_OK) return rc;
+    if ((rc = EnsureTraceScratch(ctx, R, capacity, ctx->render_overlap)) != YRH_OK) return rc;
+    if ((rc = EnsureSecondQueue(ctx, R)) != YRH_OK) return rc;
     PassView P = MakePassView(R, rd);
     P.jobs = R.b_jobs.as<DevJob>();
     P.items = R.b_items.as<DevItem>();
@@ -3235,25 +3276,6 @@ int yrh_batch_render(yrh_context* ctx, const yrh_batch_desc* d, float* job_ms, i
     P.film = R.b_film.as<yrh_film_pixel>();
     const SurfaceView S = MakeSurfaceView(R);
     const LightView L = MakeLightView(R);
-    const int max_depth = std::max(1, d->max_depth);
-    yrg::GuideView GV;
-    if ((rc = GuidePrepareView(ctx, capacity, max_depth, &GV)) != YRH_OK) return rc;
-    // Size the traversal scratch now: nothing may allocate inside a capture.
-    {
-        TraceRequest warm;
-        warm.org = P.s_org;
-        warm.dir = P.s_dir;
-        warm.n_device = BounceSlot(P.counters, 1) + kCountShadow;
-        warm.capacity = R.shadow_slots * capacity;
-        trav::TraceArgs wa;
-        int g = 0, b = 0;
-        if ((rc = PrepareTraceArgs(ctx, warm, wa, g, b)) != YRH_OK) return rc;
-        if (ctx->render_overlap) {
-            if ((rc = EnsureOverlap(ctx)) != YRH_OK) return rc;
-            warm.aux = true;
-            if ((rc = PrepareTraceArgs(ctx, warm, wa, g, b)) != YRH_OK) return rc;
-        }
-    }
     hipStream_t st = ctx->stream;
     auto launch_pass = [&]() -> int {
         int r = LaunchPassSequence(ctx, R, P, S, L, GV, capacity, max_depth, ctx->render_overlap);

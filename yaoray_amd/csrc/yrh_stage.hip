@@ -79,8 +79,9 @@ bool Pageable(const void* p) {
 
 // The context's pinned buffers (16 MiB), or null: a context's first copy
 // unless it pays for the allocation by itself (a context made for one frame
-// reads one film; 32 MiB take 1.9 ms plainly and 1.25 ms with the allocation),
-// or no memory to be had.
+// reads one film; 32 MiB into a new array take 3.2 ms plainly, 1.3 ms through
+// the buffers and 2.4 to 3.0 ms with their allocation, a process's first), or no
+// memory to be had.
 HostStage* Stage(yrh_context* ctx, size_t bytes) {
     if (ctx->stage != nullptr) return ctx->stage;
     if (!ctx->large_copy_seen && bytes < (size_t{32} << 20)) {
