@@ -11,6 +11,7 @@ import torch
 
 from yaoray_amd import Device, Scene
 from yaoray_amd import native as N
+from yaoray_amd.api import YrhError
 
 pytestmark = pytest.mark.gpu
 
@@ -153,3 +154,32 @@ def test_second_shadow_queue_follows_the_overlap_setting():
         dev.set_render_overlap(True)
         assert taken(dev, s) > 0.9 * QUEUE
         assert taken(dev, s) < 0.1 * QUEUE
+
+
+def test_recording_passes_take_no_second_shadow_queue():
+    """They wait for the Resolve of the bounce before and need the memory for
+    their records; a sampling pass of the same size then takes it."""
+    s = room()
+    with context(True) as dev:
+        guided(dev, s)
+        dev.guide_set_cell_budget(0)
+        dev.guide_set_mode(N.GUIDE_RECORD)
+        taken(dev, s)
+        dev.guide_set_mode(N.GUIDE_SAMPLE)
+        assert taken(dev, s) > 0.9 * QUEUE
+
+
+def test_second_shadow_queue_is_given_back_when_memory_is_short():
+    s = Scene.cornell(1)
+    s.build_accel()
+    with context(True) as dev:
+        dev.upload_scene(s)
+        dev.upload_shading(s)
+        taken(dev, s)
+        f0 = dev.film_read(512, 256)
+        before, total = torch.cuda.mem_get_info()
+        with pytest.raises(YrhError, match="out of memory"):
+            dev.alloc(2 * total)
+        assert torch.cuda.mem_get_info()[0] - before > 0.9 * QUEUE
+        assert taken(dev, s) > 0.9 * QUEUE
+        assert dev.film_read(512, 256).tobytes() == f0.tobytes()

@@ -22,6 +22,16 @@ int CheckHip(yrh_context* ctx, hipError_t status, const char* what) {
     return Fail(ctx, YRH_E_HIP, std::string(what) + ": " + hipGetErrorString(status));
 }
 
+int DeviceMalloc(yrh_context* ctx, void** ptr, size_t bytes, const char* what) {
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipErrorOutOfMemory && ReleaseSpareMemory(ctx)) e = hipMalloc(ptr, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the next launch's check
+        *ptr = nullptr;
+    }
+    return CheckHip(ctx, e, what);
+}
+
 int CheckStackOverflow(yrh_context* ctx) {
     if (ctx->work_counter.ptr == nullptr) return YRH_OK;
     uint32_t flag = 0;
@@ -408,7 +418,7 @@ int yrh_device_alloc(yrh_context* ctx, size_t bytes, void** out) {
     if (ctx == nullptr || out == nullptr) return YRH_E_INVALID_ARGUMENT;
     *out = nullptr;
     (void)hipSetDevice(ctx->device);
-    return CheckHip(ctx, hipMalloc(out, std::max<size_t>(bytes, 16)), "hipMalloc");
+    return DeviceMalloc(ctx, out, std::max<size_t>(bytes, 16));
 }
 
 int yrh_device_free(yrh_context* ctx, void* ptr) {
@@ -646,7 +656,7 @@ int yrh_upload_geometry(yrh_context* ctx, const yrh_geometry_desc* g) {
         std::memcpy(geo.root_lo, top.root_lo, sizeof(geo.root_lo));
         std::memcpy(geo.root_hi, top.root_hi, sizeof(geo.root_hi));
         const size_t bytes = static_cast<size_t>(std::max<int64_t>(at.units, 1)) * sizeof(float4);
-        if ((rc = CheckHip(ctx, hipMalloc(&geo.arena.ptr, bytes), "hipMalloc")) != YRH_OK) return rc;
+        if ((rc = DeviceMalloc(ctx, &geo.arena.ptr, bytes)) != YRH_OK) return rc;
         geo.arena.bytes = bytes;
         float4* base = geo.arena.as<float4>();
         if ((rc = yrh_copy_to_device(ctx, base, packed.nodes.data(), packed.nodes.size() * sizeof(DevNode))) != YRH_OK ||

@@ -95,7 +95,7 @@ int Grid(int64_t n, int block = kBlock) { return static_cast<int>(std::max<int64
 int Alloc(yrh_context* ctx, DevBuf& b, size_t bytes) {
     b.reset();
     bytes = std::max<size_t>(bytes, 16);
-    int rc = CheckHip(ctx, hipMalloc(&b.ptr, bytes), "hipMalloc");
+    int rc = DeviceMalloc(ctx, &b.ptr, bytes);
     if (rc == YRH_OK) b.bytes = bytes;
     return rc;
 }
@@ -619,10 +619,7 @@ int PackCells(yrh_context* ctx, GuideState& G) {
     if (G.cells.bytes < static_cast<size_t>(total)) {
         G.cells.reset();
         void* p = nullptr;
-        if (hipMalloc(&p, static_cast<size_t>(total)) != hipSuccess) {
-            (void)hipGetLastError();
-            return YRH_OK;
-        }
+        if (DeviceMalloc(ctx, &p, static_cast<size_t>(total)) != YRH_OK) return YRH_OK;
         G.cells.ptr = p;
         G.cells.bytes = static_cast<size_t>(total);
     }

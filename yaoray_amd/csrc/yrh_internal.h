@@ -207,6 +207,11 @@ namespace yrh {
 
 int Fail(yrh_context* ctx, int code, const std::string& message);
 int CheckHip(yrh_context* ctx, hipError_t status, const char* what);
+// hipMalloc. When memory is short, what the context holds only for speed is
+// given back first (ReleaseSpareMemory: the second shadow queue, false: there is
+// none; waits for the context's streams).
+int DeviceMalloc(yrh_context* ctx, void** ptr, size_t bytes, const char* what = "hipMalloc");
+bool ReleaseSpareMemory(yrh_context* ctx);
 // Reads (and clears) the traversal stack overflow flag after synchronising the
 // context stream: YRH_E_OVERFLOW when a traversal since the last check dropped
 // stack entries.

@@ -257,13 +257,13 @@ int OrderRaysByOrigin(yrh_context* ctx, const float4* org, int64_t n, const int3
         if (rc != YRH_OK) return rc;
         if (ctx->ray_order.bytes < order_bytes) {
             ctx->ray_order.reset();
-            rc = CheckHip(ctx, hipMalloc(&ctx->ray_order.ptr, order_bytes), "hipMalloc ray order");
+            rc = DeviceMalloc(ctx, &ctx->ray_order.ptr, order_bytes, "hipMalloc ray order");
             if (rc != YRH_OK) return rc;
             ctx->ray_order.bytes = order_bytes;
         }
         if (ctx->ray_order_scratch.bytes < scratch_bytes) {
             ctx->ray_order_scratch.reset();
-            rc = CheckHip(ctx, hipMalloc(&ctx->ray_order_scratch.ptr, scratch_bytes), "hipMalloc ray order scratch");
+            rc = DeviceMalloc(ctx, &ctx->ray_order_scratch.ptr, scratch_bytes, "hipMalloc ray order scratch");
             if (rc != YRH_OK) return rc;
             ctx->ray_order_scratch.bytes = scratch_bytes;
         }

@@ -219,7 +219,7 @@ template <typename T>
 int UploadVec(yrh_context* ctx, DevBuf& buf, const T* data, size_t count) {
     buf.reset();
     const size_t bytes = std::max<size_t>(count * sizeof(T), 16);
-    int rc = CheckHip(ctx, hipMalloc(&buf.ptr, bytes), "hipMalloc");
+    int rc = DeviceMalloc(ctx, &buf.ptr, bytes);
     if (rc != YRH_OK) return rc;
     buf.bytes = bytes;
     if (count > 0) rc = yrh_copy_to_device(ctx, buf.ptr, data, count * sizeof(T));
@@ -229,7 +229,7 @@ int UploadVec(yrh_context* ctx, DevBuf& buf, const T* data, size_t count) {
 int Alloc(yrh_context* ctx, DevBuf& buf, size_t bytes) {
     buf.reset();
     bytes = std::max<size_t>(bytes, 16);
-    int rc = CheckHip(ctx, hipMalloc(&buf.ptr, bytes), "hipMalloc");
+    int rc = DeviceMalloc(ctx, &buf.ptr, bytes);
     if (rc == YRH_OK) buf.bytes = bytes;
     return rc;
 }
@@ -2353,10 +2353,11 @@ int EnsureCapacity(yrh_context* ctx, RenderState& R, int64_t paths) {
 
 // A shadow queue of their own for odd bounces, so that Shade need not wait for
 // the Resolve just before it (LaunchPassSequence). Asked for by each overlapped
-// pass once everything else that it needs is there; given if it takes no more
-// than a quarter of the memory left.
-int EnsureSecondQueue(yrh_context* ctx, RenderState& R) {
-    if (!ctx->render_overlap || !R.second.empty()) return YRH_OK;
+// pass that does not record (those wait for that Resolve anyhow) once everything
+// else that it needs is there; given if it takes no more than a quarter of the
+// memory left, and given back when memory is short (DeviceMalloc).
+int EnsureSecondQueue(yrh_context* ctx, RenderState& R, bool recording) {
+    if (!ctx->render_overlap || recording || !R.second.empty()) return YRH_OK;
     const size_t S = static_cast<size_t>(R.cap_shadow_slots) * static_cast<size_t>(R.capacity);
     const PassArray arrays[] = {
         {&R.s_org[1], 16 * S}, {&R.s_dir[1], 16 * S}, {&R.s_li[1], 16 * S}, {&R.s_bsdf[1], 16 * S}, {&R.s_nee[1], 16 * S},
@@ -2366,10 +2367,8 @@ int EnsureSecondQueue(yrh_context* ctx, RenderState& R) {
     size_t free_bytes = 0, device_bytes = 0;
     const int rc = CheckHip(ctx, hipMemGetInfo(&free_bytes, &device_bytes), "hipMemGetInfo");
     if (rc != YRH_OK || free_bytes / 4 < bytes) return rc;
-    if (AllocPassArrays(ctx, arrays, std::size(arrays), R.second) != YRH_OK) {
-        (void)hipGetLastError();
-        R.second.clear();
-    }
+    std::vector<DevBuf> blocks;  // not R.second yet: the allocations may release that
+    if (AllocPassArrays(ctx, arrays, std::size(arrays), blocks) == YRH_OK) R.second = std::move(blocks);
     return YRH_OK;
 }
 
@@ -2740,6 +2739,14 @@ int UploadSurfaceGeometry(yrh_context* ctx, const yrh_geometry_desc* g) {
     if ((rc = UploadVec(ctx, R.spheres, sph.data(), sph.size())) != YRH_OK) return rc;
     if ((rc = UploadVec(ctx, R.sphere_info, sph_info.data(), sph_info.size())) != YRH_OK) return rc;
     return YRH_OK;
+}
+
+bool ReleaseSpareMemory(yrh_context* ctx) {
+    if (ctx->render == nullptr || ctx->render->second.empty()) return false;
+    (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->aux_stream != nullptr) (void)hipStreamSynchronize(ctx->aux_stream);
+    ctx->render->second.clear();
+    return true;
 }
 
 void DestroyRenderState(yrh_context* ctx) {
@@ -3148,7 +3155,7 @@ int yrh_render_pass(yrh_context* ctx, const yrh_render_desc* d) {
     yrg::GuideView GV;
     if ((rc = GuidePrepareView(ctx, paths, max_depth, &GV)) != YRH_OK) return rc;
     if ((rc = EnsureTraceScratch(ctx, R, paths, ctx->render_overlap)) != YRH_OK) return rc;
-    if ((rc = EnsureSecondQueue(ctx, R)) != YRH_OK) return rc;
+    if ((rc = EnsureSecondQueue(ctx, R, GV.rec != nullptr)) != YRH_OK) return rc;
     PassView P = MakePassView(R, *d);
     const SurfaceView S = MakeSurfaceView(R);
     const LightView L = MakeLightView(R);
@@ -3268,7 +3275,7 @@ int yrh_batch_render(yrh_context* ctx, const yrh_batch_desc* d, float* job_ms, i
     yrg::GuideView GV;
     if ((rc = GuidePrepareView(ctx, capacity, max_depth, &GV)) != YRH_OK) return rc;
     if ((rc = EnsureTraceScratch(ctx, R, capacity, ctx->render_overlap)) != YRH_OK) return rc;
-    if ((rc = EnsureSecondQueue(ctx, R)) != YRH_OK) return rc;
+    if ((rc = EnsureSecondQueue(ctx, R, GV.rec != nullptr)) != YRH_OK) return rc;
     PassView P = MakePassView(R, rd);
     P.jobs = R.b_jobs.as<DevJob>();
     P.items = R.b_items.as<DevItem>();

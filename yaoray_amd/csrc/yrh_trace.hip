@@ -90,7 +90,7 @@ int PrepareTraceArgs(yrh_context* ctx, const TraceRequest& r, trav::TraceArgs& a
         }
         if (rc != YRH_OK) return rc;
         spill.reset();
-        rc = CheckHip(ctx, hipMalloc(&spill.ptr, spill_bytes), "hipMalloc stack spill");
+        rc = DeviceMalloc(ctx, &spill.ptr, spill_bytes, "hipMalloc stack spill");
         if (rc != YRH_OK) return rc;
         spill.bytes = spill_bytes;
     }
