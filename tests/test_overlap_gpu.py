@@ -183,3 +183,19 @@ def test_second_shadow_queue_is_given_back_when_memory_is_short():
         assert torch.cuda.mem_get_info()[0] - before > 0.9 * QUEUE
         assert taken(dev, s) > 0.9 * QUEUE
         assert dev.film_read(512, 256).tobytes() == f0.tobytes()
+
+
+@pytest.mark.parametrize("overlap", [False, True])
+def test_suggested_pass_counts_what_the_context_holds(overlap):
+    """Half of (free memory + held path state) over the bytes of a path; with a
+    proposal and this depth below the cap, so the held bytes can be told."""
+    s, depth = Scene.cornell(1), 1000
+    s.build_accel()
+    with context(overlap) as dev:
+        guided(dev, s)
+        free = torch.cuda.mem_get_info()[0]
+        per_path = free / 2 / dev.suggest_paths_per_pass(depth)
+        grown = taken(dev, s)
+        assert grown > 0.9 * QUEUE
+        held = dev.suggest_paths_per_pass(depth) * 2 * per_path - torch.cuda.mem_get_info()[0]
+        assert 0.5 * grown < held < grown + 4 * per_path + 16 * MIB

@@ -736,6 +736,11 @@ int GuidePrepareView(yrh_context* ctx, int64_t paths, int max_depth, yrg::GuideV
     return CheckHip(ctx, hipGetLastError(), "guide view");
 }
 
+size_t GuidePassBytes(const yrh_context* ctx) {
+    const GuideState* G = ctx->guide;
+    return G == nullptr ? 0 : G->mix.bytes + G->valid.bytes + G->rec.bytes;
+}
+
 void DestroyGuideState(yrh_context* ctx) {
     delete ctx->guide;
     ctx->guide = nullptr;

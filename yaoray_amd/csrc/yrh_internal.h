@@ -273,6 +273,8 @@ void DestroyHostStage(yrh_context* ctx);
 // when no proposal is configured), sizing the per-row buffers for `paths`
 // rows and, when recording, `paths * max_depth` vertex records.
 int GuidePrepareView(yrh_context* ctx, int64_t paths, int max_depth, yrg::GuideView* view);
+// Bytes of those per-row buffers and records.
+size_t GuidePassBytes(const yrh_context* ctx);
 void DestroyGuideState(yrh_context* ctx);
 
 // Launches of the traversal kernels (yrh_trace.hip).

@@ -3121,10 +3121,14 @@ int yrh_suggest_paths_per_pass(yrh_context* ctx, int32_t max_depth, int64_t* pat
     // Per path: the path slot state (EnsureCapacity) and its shadow slots.
     const int shadow_slots = ctx->render != nullptr ? ctx->render->shadow_slots : 2;
     const bool transparent = ctx->render == nullptr || ctx->render->transparent;
-    size_t per_path = kPathSlotBytes + static_cast<size_t>(shadow_slots) *
-                                           (kShadowSlotBytes + kShadowQueueBytes + (transparent ? kWalkSlotBytes : 0));
+    const size_t per_shadow = kShadowSlotBytes + (ctx->render_overlap ? kShadowQueueBytes : 0) + (transparent ? kWalkSlotBytes : 0);
+    size_t per_path = kPathSlotBytes + static_cast<size_t>(shadow_slots) * per_shadow;
     if (ctx->guide != nullptr) per_path += kGuideRowBytes + 64 * static_cast<size_t>(std::max(1, max_depth));
-    const size_t held = ctx->render != nullptr ? static_cast<size_t>(ctx->render->capacity) * per_path : 0;
+    size_t held = GuidePassBytes(ctx);
+    if (ctx->render != nullptr) {
+        for (const DevBuf& b : ctx->render->pass) held += b.bytes;
+        for (const DevBuf& b : ctx->render->second) held += b.bytes;
+    }
     const int64_t fit = static_cast<int64_t>((free_bytes + held) / 2 / per_path);
     *paths = std::max<int64_t>(int64_t{1} << 16, std::min<int64_t>(fit, int64_t{1} << 27));
     return YRH_OK;
