@@ -11,15 +11,20 @@ pytestmark = pytest.mark.gpu
 MIB = 1 << 20
 
 
-@pytest.mark.parametrize("nbytes", [2 * MIB - 1, 2 * MIB, 2 * MIB + 1, 3 * MIB, 5 * MIB + 4093, 16 * MIB, 17 * MIB + 1,
-                                    32 * MIB, 41 * MIB + 7])
-def test_large_copies_arrive_whole(nbytes):
+# Staged from 6 MiB on, 1 MiB a chunk, a thread per two chunks up to eight.
+@pytest.mark.parametrize("nbytes", [6 * MIB - 1, 6 * MIB, 6 * MIB + 1, 7 * MIB + 4093, 9 * MIB + 1, 12 * MIB, 15 * MIB + 1,
+                                    16 * MIB, 17 * MIB + 1, 32 * MIB, 41 * MIB + 7])
+@pytest.mark.parametrize("first", [True, False])
+def test_large_copies_arrive_whole(nbytes, first):
+    """As a context's first large copy (plain under 32 MiB) and after one."""
     rng = np.random.default_rng(nbytes)
-    dev = Device(0)  # its first copy is plain unless it is very large
+    dev = Device(0)
     try:
+        if not first:
+            DeviceBuffer(dev, 32 * MIB).download(np.uint8, 32 * MIB)
         buf = DeviceBuffer(dev, nbytes + 64)
         guard = np.full(64, 7, np.uint8)
-        for _ in range(3):
+        for _ in range(1 if first else 3):
             a = rng.integers(0, 256, nbytes, np.uint8)
             buf.upload(np.concatenate([np.zeros(nbytes, np.uint8), guard]))
             buf.upload(a)
