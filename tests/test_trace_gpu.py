@@ -393,3 +393,52 @@ def test_origin_order_gives_identical_results(device, kind):
         assert np.array_equal(bb[k], aa[k]), k
     assert b["triangle"][5] == -1
     assert 0.01 < (a["triangle"] >= 0).mean() < 1.0
+
+
+def reciprocal_queries(device, z):
+    """1 / z as the triangle test computes it, and whether the slab test agrees
+    with that value as the entry distance: rays along (0, 0, z) from c = +-2^k
+    away at the triangle (0,0,0) (1,0,0) (0,1,0), whose determinant is -z. The
+    hit's t is c * fl(1/z), exact; the box, flat at z = 0, is entered at the same
+    distance, so it is met with t_max there (one triangle test) and missed with
+    the float below (none)."""
+    z = np.ascontiguousarray(z, np.float32)
+    with np.errstate(all="ignore"):
+        r = np.float32(1.0) / z
+        e = np.where(np.isfinite(r) & (r != 0.0), np.frexp(r)[1], 0)
+        c = np.copysign(np.ldexp(np.float32(1.0), np.clip(-e, -126, 126)), z).astype(np.float32)
+        at = (c * r).astype(np.float32)
+    org, d = np.full((len(z), 4), 0.25, np.float32), np.zeros((len(z), 4), np.float32)
+    org[:, 2], org[:, 3], d[:, 2] = -c, 0.0, z
+    d[:, 3] = np.inf
+    g = device.trace_closest(org, d, counters=True)
+    met, missed = d.copy(), d.copy()
+    met[:, 3], missed[:, 3] = at, np.nextafter(at, np.float32(0.0))
+    m = device.trace_closest(org, met, counters=True)["triangle_tests"]
+    n = device.trace_closest(org, missed, counters=True)["triangle_tests"]
+    return at, g, m, n
+
+
+def test_reciprocals_are_the_ieee_quotients(device):
+    """The traversal's reciprocal equals float division bit for bit: all
+    mantissas at both ends of its fast range, [2^-100, 2^100], just outside and
+    inside, both signs; zeros, subnormals, infinities and NaN as the oracle.
+    Determinants below 1e-8 are rejected whatever their reciprocal is, so
+    smaller z show in the slab test only."""
+    s = MeshArrays().add_triangles(np.array([[[0, 0, 0], [1, 0, 0], [0, 1, 0]]], np.float32)).scene()
+    s.build_accel()
+    device.upload_scene(s)
+    mantissas = np.arange(1 << 23, dtype=np.uint32)
+    for sign in (0, 1):
+        for exponent in (-101, -100, -27, -1, 0, 99, 100, 127):
+            z = (mantissas | np.uint32(exponent + 127 << 23) | np.uint32(sign << 31)).view(np.float32)
+            at, g, met, missed = reciprocal_queries(device, z)
+            assert (met == 1).all() and (missed == 0).all(), (sign, exponent)
+            if exponent >= -26:
+                assert (g["triangle"] == 0).all() and same_bits(g["t"], at), (sign, exponent)
+    special = np.array([0.0, np.inf, np.nan, 1e-45, 2.0**-149 * 3, 2.0**-127, 2.0**-126, 2.0**-101, 2.0**101, 3.4e38], np.float32)
+    z = np.tile(np.concatenate([special, -special]), 3)
+    org, d = np.full((len(z), 4), 0.25, np.float32), np.zeros((len(z), 4), np.float32)
+    org[:, 2], org[:, 3], d[:, 2], d[:, 3] = np.repeat([-1.0, 0.0, 1.0], 2 * len(special)), 0.0, z, np.inf
+    v, i, p = s.geometry()
+    assert_same(device.trace_closest(org, d, counters=True), O.trace_flat(v, i, p, s.flat_bvh(), org, d))
