@@ -199,3 +199,43 @@ def test_suggested_pass_counts_what_the_context_holds(overlap):
         assert grown > 0.9 * QUEUE
         held = dev.suggest_paths_per_pass(depth) * 2 * per_path - torch.cuda.mem_get_info()[0]
         assert 0.5 * grown < held < grown + 4 * per_path + 16 * MIB
+
+
+@pytest.mark.parametrize("overlap", [False, True])
+def test_passes_in_a_callers_graph(overlap):
+    """A pass that a caller captures after an eager one allocates nothing, each
+    replay adds what an eager pass adds, and the graph does not use the second
+    shadow queue, which the context may give back."""
+    s = Scene.cornell(1)
+    s.build_accel()
+    with context(True) as dev:
+        dev.upload_scene(s)
+        dev.upload_shading(s)
+        desc = s.render_desc(64, 48, 4, 5)
+        desc.sample_count = 4
+        dev.film_reset(64, 48)
+        for _ in range(4):
+            dev.render_pass(desc)
+        dev.synchronize()
+        eager = dev.film_read(64, 48).tobytes()
+        dev.set_render_overlap(overlap)
+        stream = torch.cuda.ExternalStream(dev._lib.yrh_stream(dev._ctx))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+            dev.render_pass(desc)
+        for turn in range(3):
+            if turn == 1:
+                with pytest.raises(YrhError, match="out of memory"):
+                    dev.alloc(2 * torch.cuda.mem_get_info()[1])
+                reuse = torch.full((16 * MIB,), 7, dtype=torch.uint8, device="cuda")
+                torch.cuda.synchronize()
+            dev.film_reset(64, 48)
+            for k in range(4):
+                if k == 2 and turn == 2:
+                    dev.render_pass(desc)
+                else:
+                    with torch.cuda.stream(stream):
+                        graph.replay()
+            dev.synchronize()
+            assert dev.film_read(64, 48).tobytes() == eager, turn
+            assert turn == 0 or bool((reuse == 7).all())

@@ -1394,8 +1394,8 @@ __device__ __forceinline__ void ShadePath(const PassView& P, const SurfaceView& 
 }
 
 template <bool kGuided, bool kAnalytic, bool kTex>
-__global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(4))) void ShadeKernel(PassView P, SurfaceView S, LightView L, yrg::GuideView G,
-                                                     int depth, int cur) {
+__global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(4))) void ShadeKernel(
+    PassView P, SurfaceView S, LightView L, yrg::GuideView G, int depth, int cur) {
     const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
     const int n = static_cast<int>(BounceSlot(P.counters, depth)[kCountQueue]);
     if (blockIdx.x == 0) {
@@ -2081,9 +2081,8 @@ __global__ void SampleValuesKernel(int kind, uint64_t seed, int spp, int64_t n, 
 
 int Grid(int64_t n, int block = kBlock) { return static_cast<int>(std::max<int64_t>(1, (n + block - 1) / block)); }
 
-// The shadow queue of bounce `depth`.
-void SetShadowQueue(const RenderState& R, PassView& P, int depth) {
-    const int k = R.second.empty() ? 0 : depth & 1;
+// Shadow queue k: 0, or the second one.
+void SetShadowQueue(const RenderState& R, PassView& P, int k) {
     P.s_org = R.s_org[k].as<float4>();
     P.s_dir = R.s_dir[k].as<float4>();
     P.s_li = R.s_li[k].as<float4>();
@@ -2281,8 +2280,11 @@ int EnsureDifferentials(yrh_context* ctx, RenderState& R) {
 }
 
 // Small pass buffers share an allocation of up to this size (freeing 30 of
-// their own costs a context made for one frame 7 ms). Not all in one: a block of
-// 1.5 GB or 256 MiB now and then takes the driver 39 ms to hand out.
+// their own costs a context made for one frame 7 ms). Not all in one: larger
+// blocks are slow to be had sooner. A context made for one 256 x 256 x 64 spp
+// frame (1.6 GB of buffers) takes 13 ms; once a process has been through about
+// 100 such frames the driver starts to hand out memory at 30 to 40 ms a frame
+// more: 6 to 13 % of 250 frames, 30 % with an allocation per array.
 constexpr size_t kPassBlockBytes = size_t{64} << 20;
 
 struct PassArray {
@@ -2352,23 +2354,33 @@ int EnsureCapacity(yrh_context* ctx, RenderState& R, int64_t paths) {
 }
 
 // A shadow queue of their own for odd bounces, so that Shade need not wait for
-// the Resolve just before it (LaunchPassSequence). Asked for by each overlapped
-// pass that does not record (those wait for that Resolve anyhow) once everything
-// else that it needs is there; given if it takes no more than a quarter of the
-// memory left, and given back when memory is short (DeviceMalloc).
-int EnsureSecondQueue(yrh_context* ctx, RenderState& R, bool recording) {
-    if (!ctx->render_overlap || recording || !R.second.empty()) return YRH_OK;
-    const size_t S = static_cast<size_t>(R.cap_shadow_slots) * static_cast<size_t>(R.capacity);
-    const PassArray arrays[] = {
-        {&R.s_org[1], 16 * S}, {&R.s_dir[1], 16 * S}, {&R.s_li[1], 16 * S}, {&R.s_bsdf[1], 16 * S}, {&R.s_nee[1], 16 * S},
-    };
-    size_t bytes = 0;
-    for (const PassArray& a : arrays) bytes += PassPadded(a.bytes);
-    size_t free_bytes = 0, device_bytes = 0;
-    const int rc = CheckHip(ctx, hipMemGetInfo(&free_bytes, &device_bytes), "hipMemGetInfo");
-    if (rc != YRH_OK || free_bytes / 4 < bytes) return rc;
-    std::vector<DevBuf> blocks;  // not R.second yet: the allocations may release that
-    if (AllocPassArrays(ctx, arrays, std::size(arrays), blocks) == YRH_OK) R.second = std::move(blocks);
+// the Resolve just before it (LaunchPassSequence): *usable says whether the pass
+// has it. Asked for by each overlapped pass that does not record (those wait for
+// that Resolve anyhow) once everything else that it needs is there; given if it
+// takes no more than a quarter of the memory left, and given back when memory is
+// short (DeviceMalloc), so a pass in a caller's graph, which may outlive it, goes
+// without.
+int EnsureSecondQueue(yrh_context* ctx, RenderState& R, bool recording, bool* usable) {
+    *usable = false;
+    if (!ctx->render_overlap || recording) return YRH_OK;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    int rc = CheckHip(ctx, hipStreamIsCapturing(ctx->stream, &capture), "hipStreamIsCapturing");
+    if (rc != YRH_OK || capture != hipStreamCaptureStatusNone) return rc;
+    if (R.second.empty()) {
+        const size_t S = static_cast<size_t>(R.cap_shadow_slots) * static_cast<size_t>(R.capacity);
+        const PassArray arrays[] = {
+            {&R.s_org[1], 16 * S}, {&R.s_dir[1], 16 * S}, {&R.s_li[1], 16 * S}, {&R.s_bsdf[1], 16 * S},
+            {&R.s_nee[1], 16 * S},
+        };
+        size_t bytes = 0;
+        for (const PassArray& a : arrays) bytes += PassPadded(a.bytes);
+        size_t free_bytes = 0, device_bytes = 0;
+        rc = CheckHip(ctx, hipMemGetInfo(&free_bytes, &device_bytes), "hipMemGetInfo");
+        if (rc != YRH_OK || free_bytes / 4 < bytes) return rc;
+        std::vector<DevBuf> blocks;  // not R.second yet, which a failing allocation releases
+        if (AllocPassArrays(ctx, arrays, std::size(arrays), blocks) == YRH_OK) R.second = std::move(blocks);
+    }
+    *usable = !R.second.empty();
     return YRH_OK;
 }
 
@@ -2408,7 +2420,7 @@ int EnsureTraceScratch(yrh_context* ctx, RenderState& R, int64_t paths, bool ove
 // Raygen and the bounces of one pass over `paths` path slots (the queue
 // capacity; the kernels read the live counts from the counter words).
 int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, const SurfaceView& S, const LightView& L,
-                       const yrg::GuideView& GV, int64_t paths, int max_depth, bool overlap) {
+                       const yrg::GuideView& GV, int64_t paths, int max_depth, bool overlap, bool two_queues) {
     hipStream_t st = ctx->stream;
     const bool guided = GV.mode != YRH_GUIDE_OFF;
     int rc;
@@ -2423,7 +2435,7 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
     hipStream_t ss = overlap ? ctx->aux_stream : st;
     hipEvent_t shaded = ctx->bounce_events[0];
     hipEvent_t* resolved = ctx->bounce_events + 1;
-    const int lag = GV.rec != nullptr || R.second.empty() ? 1 : 2;
+    const int lag = two_queues ? 2 : 1;
     {
         const StageRange r("raygen");
         hipLaunchKernelGGL(RaygenKernel, dim3(Grid(paths)), dim3(kBlock), 0, st, P);
@@ -2443,7 +2455,7 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
         tr.instance = ctx->geo.accel_kind == YRH_ACCEL_TWO_LEVEL ? P.hit_inst : nullptr;
         tr.totals = P.stats + kStatNodeTests;
         PassView Pk = P;
-        SetShadowQueue(R, Pk, depth);
+        SetShadowQueue(R, Pk, two_queues ? depth & 1 : 0);
         if (ctx->geo.accel_kind != YRH_ACCEL_TWO_LEVEL) Pk.hit_inst = nullptr;
         if (depth > 0) Pk.p_diff = nullptr;  // only camera rays carry differentials
         if (R.alpha) {
@@ -2500,7 +2512,7 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
             sr.capacity = R.shadow_slots * paths;
             sr.expected = paths;  // about one shadow ray per path in flight
             sr.work_counter = BounceSlot(P.counters, depth) + kWorkShadow;
-                sr.occluded = P.s_occ;
+            sr.occluded = P.s_occ;
             sr.totals = P.stats + kStatNodeTests;
             sr.aux = overlap;
             if ((rc = LaunchTrace(ctx, sr)) != YRH_OK) return rc;
@@ -2513,7 +2525,7 @@ int LaunchPassSequence(yrh_context* ctx, RenderState& R, const PassView& P, cons
             wr.capacity = R.shadow_slots * paths;
             wr.expected = paths;
             wr.work_counter = BounceSlot(P.counters, depth) + kWorkShadow;
-                wr.hit = P.s_trans;  // not written by the walk; LaunchTrace's checks want an output
+            wr.hit = P.s_trans;  // not written by the walk; LaunchTrace's checks want an output
             wr.totals = P.stats + kStatNodeTests;
             wr.aux = overlap;
             trav::TraceArgs wa;
@@ -3159,12 +3171,13 @@ int yrh_render_pass(yrh_context* ctx, const yrh_render_desc* d) {
     yrg::GuideView GV;
     if ((rc = GuidePrepareView(ctx, paths, max_depth, &GV)) != YRH_OK) return rc;
     if ((rc = EnsureTraceScratch(ctx, R, paths, ctx->render_overlap)) != YRH_OK) return rc;
-    if ((rc = EnsureSecondQueue(ctx, R, GV.rec != nullptr)) != YRH_OK) return rc;
+    bool two_queues = false;
+    if ((rc = EnsureSecondQueue(ctx, R, GV.rec != nullptr, &two_queues)) != YRH_OK) return rc;
     PassView P = MakePassView(R, *d);
     const SurfaceView S = MakeSurfaceView(R);
     const LightView L = MakeLightView(R);
     hipStream_t st = ctx->stream;
-    if ((rc = LaunchPassSequence(ctx, R, P, S, L, GV, paths, max_depth, ctx->render_overlap)) != YRH_OK) return rc;
+    if ((rc = LaunchPassSequence(ctx, R, P, S, L, GV, paths, max_depth, ctx->render_overlap, two_queues)) != YRH_OK) return rc;
     hipLaunchKernelGGL(AccumulateKernel, dim3(Grid(npix)), dim3(kBlock), 0, st, P);
     return CheckHip(ctx, hipGetLastError(), "render pass launch");
 }
@@ -3279,7 +3292,8 @@ int yrh_batch_render(yrh_context* ctx, const yrh_batch_desc* d, float* job_ms, i
     yrg::GuideView GV;
     if ((rc = GuidePrepareView(ctx, capacity, max_depth, &GV)) != YRH_OK) return rc;
     if ((rc = EnsureTraceScratch(ctx, R, capacity, ctx->render_overlap)) != YRH_OK) return rc;
-    if ((rc = EnsureSecondQueue(ctx, R, GV.rec != nullptr)) != YRH_OK) return rc;
+    bool two_queues = false;
+    if ((rc = EnsureSecondQueue(ctx, R, GV.rec != nullptr, &two_queues)) != YRH_OK) return rc;
     PassView P = MakePassView(R, rd);
     P.jobs = R.b_jobs.as<DevJob>();
     P.items = R.b_items.as<DevItem>();
@@ -3289,7 +3303,7 @@ int yrh_batch_render(yrh_context* ctx, const yrh_batch_desc* d, float* job_ms, i
     const LightView L = MakeLightView(R);
     hipStream_t st = ctx->stream;
     auto launch_pass = [&]() -> int {
-        int r = LaunchPassSequence(ctx, R, P, S, L, GV, capacity, max_depth, ctx->render_overlap);
+        int r = LaunchPassSequence(ctx, R, P, S, L, GV, capacity, max_depth, ctx->render_overlap, two_queues);
         if (r != YRH_OK) return r;
         for (int32_t occ = 0; occ <= max_occurrence; ++occ) {
             hipLaunchKernelGGL(AccumulateBatchKernel, dim3(Grid(capacity)), dim3(kBlock), 0, st, P, occ);
