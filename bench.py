@@ -417,7 +417,7 @@ def two_level_binding():
             out[k]["valu_lane_cycles_used"] = round(v["valu_busy"] * v["valu_lane_utilization"], 3)
     out["binding"] = ("VALU issue with a quarter of the lanes active (TLAS / instance entry / BLAS node / triangle "
                       "paths diverge within a wave) and launch tails (occupancy below the register and LDS limits); "
-                      "not HBM (L2 hit rate 0.93-0.97)")
+                      "not HBM (L2 hit rate 0.95-0.98)")
     return out
 
 

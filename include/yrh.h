@@ -540,9 +540,10 @@ int yrh_film_update_active(yrh_context* ctx, const yrh_adaptive_desc* adaptive, 
                            int64_t* converged);
 /* Paths (pixels x sample indices) one pass should hold: as many as half of
  * the device memory not in use (plus what this context's path state already
- * holds) can keep, at 360 to 800 bytes per path (more with more kinds of
- * lights, with transparent shadows; + the guiding buffers when a
- * proposal is configured), capped at 2^27. Every bounce of a pass waits for
+ * holds) can keep, at 384 to 820 bytes per path (more with more kinds of
+ * lights, with transparent shadows; 80 bytes less per kind of light with
+ * overlap off; + the guiding buffers when a proposal is configured), capped
+ * at 2^27. Every bounce of a pass waits for
  * its slowest paths, so fewer, larger passes spend less time in nearly empty
  * late bounces; the film is the same for any pass size. No counterpart in the
  * reference (its CPU passes are one sample index each). */
@@ -681,7 +682,8 @@ int yrh_set_trace_timing(yrh_context* ctx, int enable);
 int yrh_trace_phase_ms(yrh_context* ctx, float* order_ms, float* trace_ms);
 /* Render passes (yrh_render_pass) run each bounce's shadow rays on a second
  * stream, up to two bounces behind the path segments (default on; batched
- * passes too); the film is the same either way. No counterpart in the reference. */
+ * passes too; one bounce behind in recording passes and while memory is short);
+ * the film is the same either way. No counterpart in the reference. */
 int yrh_set_render_overlap(yrh_context* ctx, int enable);
 
 #if defined(__GNUC__)

@@ -26,13 +26,14 @@
 // levels in a per-lane global region; one pending sibling per level fits its
 // capacity, max_depth + 2.
 //
-// What bounds it: instruction issue (VALU busy 1.0 on 1 M triangles, 0.73
-// instanced, with 0.29-0.37 of the lanes active) and, as much, the lanes' own
-// 16-byte record requests (TD busy 0.9-1.0). One-register records, an
-// end-of-leaf mark in the slot, constant-stride stack addresses and no
-// per-rejection branches in the triangle test took 8.39 M rays on 1 M
-// triangles from 4.15 to 3.81 ms a call, 1.29 M rays on 2000 instances from
-// 437 to 333 us, the instanced 1080p x 16 spp frame from 190 to 144 ms.
+// What bounds it: instruction issue (VALU busy 0.94 with 0.37 of the lanes
+// active for 8.39 M rays on 1 M triangles, 1.0 and 0.25 for the instanced 1080p
+// frame) and, as much, the lanes' own 16-byte record requests (TD busy 0.95 and
+// 0.94). One-register records, an end-of-leaf mark in the slot, constant-stride
+// stack addresses and no per-rejection branches in the triangle test took the
+// 1 M-triangle cast from 4.15 to 3.81 ms a call, 1.29 M rays on 2000 instances
+// from 437 to 333 us (three contexts' calls in flight), the frame at 16 spp from
+// 190 to 144 ms.
 //
 // A policy object supplies each ray's first segment (Begin) and receives each
 // finished segment with its origin and direction (Finish); Finish may hand
@@ -99,8 +100,9 @@ __device__ __forceinline__ uint64_t Ballot(bool p) { return __builtin_amdgcn_bal
 // FMA on the hardware reciprocal (P. Markstein, "Computation of elementary
 // functions on the IBM RISC System/6000 processor", 1990), 5 instructions
 // against the 11 of the general division. Equal to it for every |x| in
-// [2^-100, 2^100] (all 3.4e9 values compared on the GPU); a wave with a lane
-// outside (zero, infinite and NaN included) runs the general division too.
+// [2^-100, 2^100] (tests/test_trace_gpu.py: every mantissa at the ends of the
+// range and in between); a wave with a lane outside (zero, infinite and NaN
+// included) runs the general division too.
 // `below`: values under 2^-100 occur (else their result is not used).
 template <bool below>
 __device__ __forceinline__ float Reciprocal(float x) {
@@ -443,14 +445,15 @@ struct RayArrayPolicy {
 //
 // A queue with at most 64 rays per wave is dealt out by position: no atomic,
 // and the rays lie on spread_waves waves (two per SIMD) if they can, so a small
-// queue runs at the latency of few lanes per wave (4096 rays on 20 k triangles:
-// 139 us in full waves, 105, 96, 91 and 90 us on 1, 2, 4 and 8 waves per SIMD;
-// the short bounces of a Cornell frame pay for the extra waves, 2.14, 2.14,
-// 2.23 and 2.69 ms; 8 instanced cameras 48.2, 46.2, 45.4, 47.2 ms). A longer one keeps a counter per stretch; a wave claims
-// as many rays as it has idle lanes with one atomic and moves on to the next
-// stretch when its own is used up. (Dealing the first 64 by position there too
-// cost 1.29 M instanced rays 569 -> 606 us, and reading the counters before
-// moving on cost 8.39 M rays 4.1 -> 4.8 ms.)
+// queue runs at the latency of few lanes per wave. 4096 rays on 20 k triangles,
+// one context's calls one after another: 310 us at 4 rays a lane, 103, 93, 88
+// and 90 us on 1, 2, 4 and 8 waves per SIMD; the short bounces of a Cornell
+// frame pay for the extra waves, 2.00, 1.73, 1.73, 1.80 and 2.17 ms; 8 instanced
+// cameras 48.8, 37.5, 36.0, 36.0 and 37.0 ms. A longer queue keeps a counter per
+// stretch; a wave claims as many rays as it has idle lanes with one atomic and
+// moves on to the next stretch when its own is used up. (Dealing the first 64 by
+// position there too cost 1.29 M instanced rays 569 -> 606 us, and reading the
+// counters before moving on cost 8.39 M rays 4.1 -> 4.8 ms.)
 struct RaySource {
     int part;          // the stretch this wave claims from
     int parts_left;    // stretches not yet found used up (0: dealt by position)
