@@ -82,10 +82,12 @@ def test_gradients_match_bf16_oracle(device):
     assert np.all(gm[10240:].reshape(64, 48)[:, 40:] == 0.0)
 
 
-@pytest.mark.parametrize("log2,rmin,rmax,rows", [(17, 40, 64, 700), (14, 2, 12, 2100), (16, 8, 256, 4100), (12, 16, 64, 16)])
+@pytest.mark.parametrize("log2,rmin,rmax,rows", [(17, 40, 64, 700), (14, 2, 12, 2100), (16, 8, 256, 4100), (12, 16, 64, 16),
+                                                 (17, 40, 64, 2100), (14, 2, 12, 2047), (14, 2, 12, 2048)])
 def test_gradients_with_any_number_of_copied_levels(device, log2, rmin, rmax, rows):
     """No level, every level and some levels added through the per-workgroup
-    copies; a second call starts from cleared copies. Tolerances: bf16 products,
+    copies, which batches of 2048 rows and more use; a second call starts from
+    cleared copies. Tolerances: bf16 products,
     FP32 sums in another order, as in test_gradients_match_bf16_oracle."""
     d = guide_desc(log2, rmin, rmax)
     configure(device, d)

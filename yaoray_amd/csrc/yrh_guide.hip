@@ -44,6 +44,10 @@ constexpr int64_t kGuideCellBudgetDefault = static_cast<int64_t>(512) << 20;
 constexpr int kReplicas = 32;
 constexpr int kReplicaHeader = 32;          // words: [0] loss, the rest unused (a cache line)
 constexpr int64_t kCoarseEntries = 1 << 15;  // entries of the levels that are copied, at most
+// Rows from which the copies pay for the fold. A training step with a table of
+// 2^16 entries, copied / not: 500 rows 62 / 56 us, 2000 72 / 70, 3000 74 / 78,
+// 8192 100 / 125; with 2^12 entries 58 / 52, 68 / 68, 70 / 76, 101 / 128.
+constexpr int64_t kCopyRows = 2048;
 struct CoarseGrid {
     int32_t levels = 0;                      // levels 0 .. levels - 1 are copied
     int32_t begin[yrg::kGuideLevels + 1] = {};  // their first entries
@@ -173,7 +177,7 @@ struct TrainArgs {
     const bf16x4_t* bwd;
     const float2* table;
     float* table_grad;
-    float* replicas;
+    float* replicas;    // or the loss itself: no levels are copied and the stride is 0
     CoarseGrid coarse;
     yrg::GuideGrid grid;
     uint16_t* act;
@@ -662,14 +666,18 @@ int BackwardPass(yrh_context* ctx, GuideState& G, const float4* samples, const u
     A.bwd = G.frag_bwd.as<bf16x4_t>();
     A.table = G.table.as<float2>();
     A.table_grad = G.table_grad.as<float>();
-    A.replicas = G.replicas.as<float>();
+    const bool copies = rows >= kCopyRows;
+    A.replicas = copies ? G.replicas.as<float>() : loss;
     A.coarse = G.coarse;
+    if (!copies) A.coarse.levels = A.coarse.stride = 0;
     A.grid = G.grid;
     A.act = G.act.as<uint16_t>();
     A.grad = G.grad.as<uint16_t>();
     hipLaunchKernelGGL(GuideBackwardKernel, dim3(Grid(nrb, 4)), dim3(kBlock), 0, ctx->stream, A);
-    hipLaunchKernelGGL(GuideFoldKernel, dim3(Grid(G.coarse.stride)), dim3(kBlock), 0, ctx->stream, G.replicas.as<float>(),
-                       G.coarse, G.table_grad.as<float>(), G.grid.table_size, loss);
+    if (copies) {
+        hipLaunchKernelGGL(GuideFoldKernel, dim3(Grid(G.coarse.stride)), dim3(kBlock), 0, ctx->stream,
+                           G.replicas.as<float>(), G.coarse, G.table_grad.as<float>(), G.grid.table_size, loss);
+    }
     hipLaunchKernelGGL(GuideWeightGradKernel, dim3(Grid(kTiles * chunks, 4)), dim3(kBlock), 0, ctx->stream,
                        G.act.as<uint16_t>(), G.grad.as<uint16_t>(), nrb, chunks, G.partial.as<float>());
     return CheckHip(ctx, hipGetLastError(), "guide backward");
