@@ -629,7 +629,7 @@ def bench_guiding(dev, width, height, ref_spp, spp_list, train_passes, train_ste
             "unit": "TFLOP/s (BF16 MFMA, FP32 accumulation)",
             "frac": round(tflops / 2500.0, 5),
             "bound": "not MFMA: the hash-grid gradient's atomic adds and the latency of one wave per 16 samples "
-                     "(2 waves per SIMD); the matrix products are a few percent of the step",
+                     "(1 wave per SIMD at 16384 samples); the matrix products are a few percent of the step",
             "timing": "HIP events on the context stream around each yrh_guide_train call, inside the guided clock",
         }
     px = [p["seconds"] for p in plain]

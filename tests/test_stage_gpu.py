@@ -63,7 +63,7 @@ def test_uploads_cost_no_more_than_a_plain_copy(mib):
         buf.free()
     finally:
         dev.close()
-    assert np.median(ours) < 1.15 * np.median(plain)
+    assert np.percentile(ours, 25) < 1.15 * np.percentile(plain, 25)
 
 
 def test_destinations_that_are_not_pageable(device):
@@ -91,4 +91,4 @@ def test_destinations_that_are_not_pageable(device):
         torch.cuda.synchronize()
         plain.append(time.perf_counter() - t0)
     buf.free()
-    assert np.median(ours) < 1.3 * np.median(plain)
+    assert np.percentile(ours, 25) < 1.3 * np.percentile(plain, 25)
